@@ -32,11 +32,12 @@
 //
 // Small outputs with a long K (weight gradients) are split along K into f32
 // partial tiles in a caller workspace and summed (bias/beta/cast fused) by
-// a second pass.  f32 inputs use a plain 64x64 register-tiled FMA kernel.
+// a second pass.  f32 inputs: gemm_f32.hip.
 #include <stdio.h>
 #include <stdlib.h>
 
 #include "common.h"
+#include "gemm.h"
 #include "mfma.h"
 
 #ifndef GEMM_XCD_FLAT
@@ -51,47 +52,9 @@ namespace {
 
 constexpr int kCUs = 256;
 
-struct GemmArgs {
-  void* c;
-  int c_dt;
-  int64_t c_rs, c_bs;
-  const void* a;
-  int64_t a_rs, a_cs, a_bs;
-  const void* b;
-  int64_t b_rs, b_cs, b_bs;
-  const void* bias;
-  int bias_dt;
-  int beta;
-  int64_t m, n, k;
-  float* part;     // split-K partials [splits][batch][m][n] (f32) or null
-  int64_t kchunk;  // K per split
-  int tiles_n;     // tiles along n
-  int batch;       // batch count (grid.y = splits * batch)
-  int ab_dt;       // operand dtype (for rounding through it)
-  int round_c;     // round C (and the row sums) through ab_dt before storing
-  void* rowsum;    // optional sum over k of A's rows [batch][m], or null
-  int rowsum_dt;
-  float* rs_part;  // split-K row-sum partials [splits * rs_slots][batch][m]
-};
-
 // v rounded to the 16-bit operand dtype and widened back.
 __device__ __forceinline__ float round_through(float v, int dt) {
   return dt == MI355X_BF16 ? (float)(bf16)v : (float)(f16)v;
-}
-
-__device__ __forceinline__ float ld_any(const void* p, int dt, int64_t i) {
-  switch (dt) {
-    case MI355X_F32: return ((const float*)p)[i];
-    case MI355X_BF16: return (float)((const bf16*)p)[i];
-    default: return (float)((const f16*)p)[i];
-  }
-}
-__device__ __forceinline__ void st_any(void* p, int dt, int64_t i, float v) {
-  switch (dt) {
-    case MI355X_F32: ((float*)p)[i] = v; break;
-    case MI355X_BF16: ((bf16*)p)[i] = (bf16)v; break;
-    default: ((f16*)p)[i] = (f16)v; break;
-  }
 }
 
 // Sum split-K partials: C = sum_s part[s] (+bias) (+C).
@@ -808,55 +771,6 @@ __global__ void __launch_bounds__(256) pack_k_contig_v8(uint16_t* __restrict__ d
 }
 
 // ---------------------------------------------------------------------------
-// f32: 64x64 tile, 256 threads, 4x4 outputs per thread.
-// ---------------------------------------------------------------------------
-__global__ void __launch_bounds__(256) gemm_f32(GemmArgs g) {
-  __shared__ float As[16][64 + 4];
-  __shared__ float Bs[16][64 + 4];
-  const int64_t batch = blockIdx.z;
-  const int64_t m0 = (int64_t)blockIdx.y * 64, n0 = (int64_t)blockIdx.x * 64;
-  const float* A = (const float*)g.a + batch * g.a_bs;
-  const float* B = (const float*)g.b + batch * g.b_bs;
-  const int tx = threadIdx.x & 15, ty = threadIdx.x >> 4;
-  float acc[4][4] = {};
-  for (int64_t k0 = 0; k0 < g.k; k0 += 16) {
-    for (int e = threadIdx.x; e < 16 * 64; e += 256) {
-      const int kk = e / 64, r = e % 64;
-      const int64_t gm = m0 + r, gk = k0 + kk, gn = n0 + r;
-      As[kk][r] = (gm < g.m && gk < g.k) ? A[gm * g.a_rs + gk * g.a_cs] : 0.f;
-      Bs[kk][r] = (gn < g.n && gk < g.k) ? B[gk * g.b_rs + gn * g.b_cs] : 0.f;
-    }
-    __syncthreads();
-#pragma unroll
-    for (int kk = 0; kk < 16; ++kk) {
-      float a[4], b[4];
-#pragma unroll
-      for (int i = 0; i < 4; ++i) a[i] = As[kk][ty * 4 + i], b[i] = Bs[kk][tx * 4 + i];
-#pragma unroll
-      for (int i = 0; i < 4; ++i)
-#pragma unroll
-        for (int j = 0; j < 4; ++j) acc[i][j] += a[i] * b[j];
-    }
-    __syncthreads();
-  }
-  void* Cb = (char*)g.c + batch * g.c_bs * (g.c_dt == MI355X_F32 ? 4 : 2);
-#pragma unroll
-  for (int i = 0; i < 4; ++i) {
-    const int64_t row = m0 + ty * 4 + i;
-    if (row >= g.m) continue;
-#pragma unroll
-    for (int j = 0; j < 4; ++j) {
-      const int64_t col = n0 + tx * 4 + j;
-      if (col >= g.n) continue;
-      float v = acc[i][j] + (g.bias ? ld_any(g.bias, g.bias_dt, col) : 0.f);
-      const int64_t off = row * g.c_rs + col;
-      if (g.beta) v += ld_any(Cb, g.c_dt, off);
-      st_any(Cb, g.c_dt, off, v);
-    }
-  }
-}
-
-// ---------------------------------------------------------------------------
 // planning
 // ---------------------------------------------------------------------------
 struct Plan {
@@ -994,6 +908,8 @@ int launch_tile(GemmArgs g, int64_t batch, int splits, hipStream_t s) {
   return launch_layout<T, CFG, KT, false>(g, grid, s);
 }
 
+}  // namespace
+
 // Sum the split-K partials into C and, with rs_slots > 0, the row-sum
 // partials into the row sums; returns -1 when the C sum needs the scalar
 // kernel (then the caller sums the row sums itself).
@@ -1027,6 +943,8 @@ int splitk_finish(const GemmArgs& g, int64_t batch, int splits, int rs_slots, hi
   const int rc = check_launch("mi355x_gemm splitk_reduce");
   return rc ? rc : -1;
 }
+
+namespace {
 
 template <typename T>
 int launch_mfma(GemmArgs g, int64_t batch, const Plan& p, hipStream_t s) {
@@ -1125,7 +1043,8 @@ extern "C" int64_t mi355x_gemm_workspace_bytes(const void* a, int64_t a_rs, int6
                                                int64_t a_bs, const void* b, int64_t b_rs,
                                                int64_t b_cs, int64_t b_bs, int ab_dtype,
                                                int64_t batch, int64_t m, int64_t n, int64_t k) {
-  if (ab_dtype == MI355X_F32 || m <= 0 || n <= 0 || k <= 0) return 0;
+  if (m <= 0 || n <= 0 || k <= 0) return 0;
+  if (ab_dtype == MI355X_F32) return gemm_f32_workspace(batch, m, n, k);
   return ws_layout(batch, m, n, k, a, a_rs, a_cs, a_bs, b, b_rs, b_cs, b_bs).total;
 }
 
@@ -1154,9 +1073,7 @@ extern "C" int mi355x_gemm_ex(void* c, int c_dtype, int64_t c_rs, int64_t c_bs, 
              beta, m, n, k, nullptr, k, 1, 1, ab_dtype, round_c, a_rowsum, a_rowsum_dtype, nullptr};
   if (ab_dtype == MI355X_F32) {
     MI_REQUIRE(!a_rowsum && !round_c, "mi355x_gemm: row sums and ROUND need 16-bit operands");
-    dim3 grid(ceil_div(n, 64), ceil_div(m, 64), (unsigned)batch);
-    gemm_f32<<<grid, 256, 0, s>>>(g);
-    return check_launch("mi355x_gemm");
+    return gemm_f32_launch(g, batch, workspace, ws_bytes, s);
   }
   WsLayout w = ws_layout(batch, m, n, k, a, a_rs, a_cs, a_bs, b, b_rs, b_cs, b_bs);
   MI_REQUIRE(batch * w.plan.splits < 65536, "mi355x_gemm: batch x splits too large");
