@@ -318,6 +318,12 @@ int mi355x_layer_norm_fwd_ex(void* y, void* y_low, int low_dtype, float* mean,
                              float* rstd, const void* x, const void* gamma,
                              const void* beta, int64_t rows, int64_t cols,
                              double eps, int dtype, mi355x_stream_t stream);
+/* mi355x_layer_norm_fwd for bf16/f16 rows, with mean and rstd stored in the
+ * row type (what ATen's native_layer_norm returns for such rows) by the same
+ * kernel: no cast of each behind it.  Computed in f32 either way. */
+int mi355x_layer_norm_fwd_low(void* y, void* mean, void* rstd, const void* x, const void* gamma,
+                              const void* beta, int64_t rows, int64_t cols, double eps, int dtype,
+                              mi355x_stream_t stream);
 /* The residual add of a pre-LayerNorm block fused into the norm that reads
  * it: x_out = a + r (a f32, r f32/bf16/f16, summed in f32 exactly as a
  * separate add would), then y = LayerNorm(x_out) with y_low as in

@@ -260,6 +260,13 @@ class HostStandIn:
             dense(_val(y_low), DT[low_dt], (rows, cols)).copy_(self.last_ln_y)
         return 0
 
+    def mi355x_layer_norm_fwd_low(self, y, mean, rstd, x, g, b, rows, cols, eps, dt, stream):
+        stats = [torch.empty(rows) for _ in range(2)]
+        self.mi355x_layer_norm_fwd(y, stats[0].data_ptr(), stats[1].data_ptr(), x, g, b, rows, cols, eps, dt, stream)
+        for ptr, v in zip((mean, rstd), stats):
+            dense(_val(ptr), DT[dt], (rows,)).copy_(v)
+        return 0
+
     def mi355x_add_cast(self, out, low, low_dt, a, r, r_dt, n, stream):
         self.add_cast_calls = getattr(self, "add_cast_calls", 0) + 1
         A = dense(_val(a), torch.float32, (n,))

@@ -31,11 +31,19 @@ __device__ __forceinline__ float ln_out(float x, float mu, float r, float g, flo
   return (x - mu) * r * g + b;
 }
 
+// A row's statistics, in f32 or (LOW) in the row type, as ATen returns them
+// for 16-bit rows.
+template <typename T, bool LOW>
+__device__ __forceinline__ void st_stats(float* mean, float* rstd, int64_t row, float mu, float r) {
+  if (mean) { if (LOW) ((T*)mean)[row] = from_f32<T>(mu); else mean[row] = mu; }
+  if (rstd) { if (LOW) ((T*)rstd)[row] = from_f32<T>(r); else rstd[row] = r; }
+}
+
 // y (optional when y_low is given) and y_low (optional, element type TL): a
 // second copy of y rounded to a 16-bit type, the operand an autocast matmul
 // consumes next.  A caller that needs only the 16-bit copy passes y = null
 // and can produce y later with mi355x_layer_norm_apply.
-template <typename T, typename TL, int NV>
+template <typename T, typename TL, int NV, bool LOW>
 __global__ void __launch_bounds__(kThreads)
     ln_fwd_wave(T* __restrict__ y, TL* __restrict__ y_low, float* __restrict__ mean_out,
                 float* __restrict__ rstd_out, const T* __restrict__ x, const T* __restrict__ gamma,
@@ -86,10 +94,7 @@ __global__ void __launch_bounds__(kThreads)
       if (y_low) Vec4<TL>::store(y_low + row * cols + c, o);
     }
   }
-  if (lane == 0) {
-    if (mean_out) mean_out[row] = mu;
-    if (rstd_out) rstd_out[row] = r;
-  }
+  if (lane == 0) st_stats<T, LOW>(mean_out, rstd_out, row, mu, r);
 }
 
 // The residual add fused in front of the norm: x = a + r (r of type TR,
@@ -160,7 +165,7 @@ __global__ void __launch_bounds__(kThreads)
 }
 
 // Any `cols`: one block per row, three passes over the row.
-template <typename T, typename TL>
+template <typename T, typename TL, bool LOW>
 __global__ void __launch_bounds__(kThreads)
     ln_fwd_block(T* __restrict__ y, TL* __restrict__ y_low, float* __restrict__ mean_out,
                  float* __restrict__ rstd_out, const T* __restrict__ x, const T* __restrict__ gamma,
@@ -183,10 +188,7 @@ __global__ void __launch_bounds__(kThreads)
     if (y) y[row * cols + c] = from_f32<T>(o);
     if (y_low) y_low[row * cols + c] = from_f32<TL>(o);
   }
-  if (threadIdx.x == 0) {
-    if (mean_out) mean_out[row] = mu;
-    if (rstd_out) rstd_out[row] = r;
-  }
+  if (threadIdx.x == 0) st_stats<T, LOW>(mean_out, rstd_out, row, mu, r);
 }
 
 // y from x and the statistics a forward saved (mean, rstd per row): the
@@ -527,7 +529,7 @@ int bwd_blocks(int64_t rows) {
   return rows > 0 ? (int)((rows + rpb - 1) / rpb) : 1;
 }
 
-template <typename T, typename TL>
+template <typename T, typename TL, bool LOW = false>
 int fwd_impl(T* y, TL* y_low, float* mean, float* rstd, const T* x, const T* g, const T* b, int64_t rows,
              int64_t cols, float eps, hipStream_t s) {
   const size_t al = 4 * sizeof(T);
@@ -536,14 +538,14 @@ int fwd_impl(T* y, TL* y_low, float* mean, float* rstd, const T* x, const T* g, 
   const unsigned grid = ceil_div(rows, kWaves);
   switch (nv) {
 #define LN_FWD_CASE(V) \
-    case V: ln_fwd_wave<T, TL, V><<<grid, kThreads, 0, s>>>(y, y_low, mean, rstd, x, g, b, rows, (int)cols, eps); break;
+    case V: ln_fwd_wave<T, TL, V, LOW><<<grid, kThreads, 0, s>>>(y, y_low, mean, rstd, x, g, b, rows, (int)cols, eps); break;
     LN_FWD_CASE(1)
     LN_FWD_CASE(2)
     LN_FWD_CASE(3)
     LN_FWD_CASE(4)
     LN_FWD_CASE(8)
 #undef LN_FWD_CASE
-    default: ln_fwd_block<T, TL><<<(unsigned)rows, kThreads, 0, s>>>(y, y_low, mean, rstd, x, g, b, rows, cols, eps);
+    default: ln_fwd_block<T, TL, LOW><<<(unsigned)rows, kThreads, 0, s>>>(y, y_low, mean, rstd, x, g, b, rows, cols, eps);
   }
   return check_launch("mi355x_layer_norm_fwd");
 }
@@ -734,6 +736,23 @@ extern "C" int mi355x_layer_norm_fwd_ex(void* y, void* y_low, int low_dtype, flo
                                 (const f16*)beta, rows, cols, (float)eps, s);
   }
   return fail(MI355X_EUNSUPPORTED, "mi355x_layer_norm_fwd: unsupported dtype %d", dtype);
+}
+
+extern "C" int mi355x_layer_norm_fwd_low(void* y, void* mean, void* rstd, const void* x, const void* gamma,
+                                         const void* beta, int64_t rows, int64_t cols, double eps, int dtype,
+                                         mi355x_stream_t stream) {
+  MI_REQUIRE(rows >= 0 && cols > 0, "mi355x_layer_norm_fwd_low: bad shape [%lld, %lld]", (long long)rows,
+             (long long)cols);
+  if (rows == 0) return MI355X_OK;
+  MI_REQUIRE(x && y, "mi355x_layer_norm_fwd_low: null pointer");
+  hipStream_t s = (hipStream_t)stream;
+  if (dtype == MI355X_BF16)
+    return fwd_impl<bf16, bf16, true>((bf16*)y, nullptr, (float*)mean, (float*)rstd, (const bf16*)x,
+                                      (const bf16*)gamma, (const bf16*)beta, rows, cols, (float)eps, s);
+  if (dtype == MI355X_F16)
+    return fwd_impl<f16, f16, true>((f16*)y, nullptr, (float*)mean, (float*)rstd, (const f16*)x, (const f16*)gamma,
+                                    (const f16*)beta, rows, cols, (float)eps, s);
+  return fail(MI355X_EUNSUPPORTED, "mi355x_layer_norm_fwd_low: bf16 or f16 rows (got dtype %d)", dtype);
 }
 
 extern "C" int mi355x_layer_norm_fwd_add(void* y, void* y_low, int low_dtype, float* mean, float* rstd,

@@ -1737,11 +1737,22 @@ def fast_aten_native_layer_norm(input, normalized_shape, weight, bias, eps):
     b = None if b is None else (_contig(b) if b._dtype == a._dtype else materialize_contiguous(b, a._dtype))
     out = _alloc(a._shape, a._dtype, a._device)
     stat_shape = tuple(a._shape[:-k]) + (1,) * k
-    mean = _alloc(stat_shape, torch.float32, a._device)
-    rstd = _alloc(stat_shape, torch.float32, a._device)
+    # ATen returns the statistics in the input dtype (aten_fast.py:5228-5245)
+    mean = _alloc(stat_shape, a._dtype, a._device)
+    rstd = _alloc(stat_shape, a._dtype, a._device)
+    if a._dtype != torch.float32:
+        if rows and cols:
+            check(
+                "mi355x_layer_norm_fwd_low",
+                lib().mi355x_layer_norm_fwd_low(
+                    out._ptr, mean._ptr, rstd._ptr, x._ptr, g._ptr if g is not None else None,
+                    b._ptr if b is not None else None, rows, cols, float(eps), _code(a._dtype), _STREAM,
+                ),
+            )
+        return out, mean, rstd
     # Under autocast an f32 layer norm feeds a lower-precision matmul: the
     # kernel also writes y in that dtype, which the cast then takes.
-    low_dt = _autocast_low_dtype() if a._dtype == torch.float32 else None
+    low_dt = _autocast_low_dtype()
     low = _alloc(a._shape, low_dt, a._device) if (low_dt is not None and rows and cols) else None
     # With the 16-bit copy written, the f32 y is left to a lazy launch: in an
     # autocast step only the copy is read (the next linear takes it).
@@ -1779,10 +1790,6 @@ def fast_aten_native_layer_norm(input, normalized_shape, weight, bias, eps):
                 b._ptr if b is not None else None, rows, cols, code, _STREAM))
 
         lazy(out, [t for t in (x, mean, rstd, g, b) if t is not None], fill)
-    if a._dtype != torch.float32:
-        # ATen returns the statistics in the input dtype (aten_fast.py:5228-5245)
-        mean = materialize_contiguous(mean, a._dtype)
-        rstd = materialize_contiguous(rstd, a._dtype)
     return out, mean, rstd
 
 
