@@ -28,6 +28,11 @@ struct GemmArgs {
   float* rs_part;  // split-K row-sum partials [splits * rs_slots][batch][m]
 };
 
+// v rounded to the 16-bit operand dtype and widened back.
+__device__ __forceinline__ float round_through(float v, int dt) {
+  return dt == MI355X_BF16 ? (float)(bf16)v : (float)(f16)v;
+}
+
 __device__ __forceinline__ float ld_any(const void* p, int dt, int64_t i) {
   switch (dt) {
     case MI355X_F32: return ((const float*)p)[i];
@@ -47,6 +52,15 @@ __device__ __forceinline__ void st_any(void* p, int dt, int64_t i, float v) {
 // rs_slots > 0 the row sums too.  Returns -1 when C is done by the scalar
 // kernel, which leaves the row sums to the caller.
 int splitk_finish(const GemmArgs& g, int64_t batch, int splits, int rs_slots, hipStream_t s);
+
+// One launch of the 16-bit MFMA tiles (gemm_tile.h) in block configuration
+// `cfg`; KT: K is not a multiple of 64.
+template <typename T, bool KT>
+int gemm_tiles(const GemmArgs& g, int64_t batch, int cfg, int splits, hipStream_t s);
+extern template int gemm_tiles<bf16, false>(const GemmArgs&, int64_t, int, int, hipStream_t);
+extern template int gemm_tiles<bf16, true>(const GemmArgs&, int64_t, int, int, hipStream_t);
+extern template int gemm_tiles<f16, false>(const GemmArgs&, int64_t, int, int, hipStream_t);
+extern template int gemm_tiles<f16, true>(const GemmArgs&, int64_t, int, int, hipStream_t);
 
 // f32 operands (gemm_f32.hip): bytes of split-K partials that the call can
 // use, and the launch, which runs without splits when it has no workspace.

@@ -1,34 +1,8 @@
 // GEMM: C[b] = A[b] * B[b] (+ bias row) (+ C if beta), f32 accumulation.
 //
-// bf16/f16 inputs run on MFMA (v_mfma_f32_16x16x32_*).  One kernel template
-// covers every layout of the training GEMMs:
-//   fwd  x*W^T : A k-contiguous, B k-contiguous (W rows)
-//   dX   dY*W  : A k-contiguous, B n-contiguous
-//   dW   dY^T*X: A m-contiguous, B n-contiguous
-// Operand tiles (64 k per step) go global -> LDS directly with
-// global_load_lds_dwordx4 (each wave instruction fills 1 KB, lane i writing
-// bytes [16i, 16i+16)), two stages deep: the next step's loads are issued
-// right after the barrier and stream in under the current step's MFMAs.
-//   k-contiguous tile: [row][64 k] rows of 128 bytes, 16-byte chunks
-//     XOR-swizzled by (row >> 1) & 7 so a fragment read of 16 rows hits 16
-//     distinct bank groups;
-//   m/n-contiguous tile: [k][rows] with chunks swizzled by kswz(k); fragments
-//     are read transposed with ds_read_b64_tr_b16.
-// A lane's global source address is chosen so that its fixed LDS slot
-// receives the swizzled chunk, so staging costs no registers.
-//
-// Three block configurations (waves arranged WGM x WGN, each wave owning a
-// (BM/WGM) x (BN/WGN) sub-tile of 16x16 MFMA tiles):
-//   C128: 128x128, 4 waves of 64x64, 64 KB LDS, two blocks per CU;
-//   C192: 128x192, 4 waves of 64x96, 80 KB LDS, two blocks per CU (B
-//         k-contiguous only); N = 768, 2304, 3072 split into whole rounds;
-//   C256: 256x256, 8 waves of 128x64, 128 KB LDS, one block per CU (fewer
-//         LDS bytes per flop; preferred when its tiles fill the CUs evenly).
-// The block -> tile map is XCD-aware (the hardware deals workgroups to the 8
-// XCDs round-robin): each XCD walks a contiguous run of tiles, so the blocks
-// sharing an L2 share operand panels.  Index math is 32-bit and the edge
-// clamps are folded into per-thread base pointers once, so the prologue
-// stays short next to a K = 768 main loop.
+// This file plans a call: which block configuration of the 16-bit MFMA tiles
+// (gemm_tile.h), packed copies of operands that cannot be read in place, and
+// K splits, whose partials it sums.
 //
 // Small outputs with a long K (weight gradients) are split along K into f32
 // partial tiles in a caller workspace and summed (bias/beta/cast fused) by
@@ -38,24 +12,12 @@
 
 #include "common.h"
 #include "gemm.h"
-#include "mfma.h"
-
-#ifndef GEMM_XCD_FLAT
-#define GEMM_XCD_FLAT 1
-#endif
 #include "vec.h"
-
-extern __shared__ __attribute__((aligned(16))) char gemm_smem[];
 
 namespace mi {
 namespace {
 
 constexpr int kCUs = 256;
-
-// v rounded to the 16-bit operand dtype and widened back.
-__device__ __forceinline__ float round_through(float v, int dt) {
-  return dt == MI355X_BF16 ? (float)(bf16)v : (float)(f16)v;
-}
 
 // Sum split-K partials: C = sum_s part[s] (+bias) (+C).
 __global__ void __launch_bounds__(256) splitk_reduce(GemmArgs g, int splits, int64_t nb) {
@@ -162,524 +124,6 @@ __global__ void __launch_bounds__(256) splitk_rowsum_reduce(GemmArgs g, int spli
   else rowsum_reduce_body(g, slots, nb, blockIdx.x - nbc, gridDim.x - nbc);
 }
 
-// Row swizzle of a k-contiguous tile with BK-element (2*BK-byte) rows: row r
-// stores its 16-byte chunk c in slot c ^ rswz(r).  A fragment read (16 rows
-// at one chunk) then covers every bank once: BK = 64, 8 chunks, rows paired
-// by (r >> 1); BK = 32, 4 chunks, rows grouped by (r >> 2).
-template <int BK>
-__device__ __forceinline__ int rswz(int r) { return BK == 64 ? ((r >> 1) & 7) : ((r >> 2) & 3); }
-
-// k-contiguous operand tile: ROWS rows x BK k, loaded by NT threads, one
-// 1 KB instruction per RPI rows.  Thread (wave w, lane l) handles rows
-// r = RPI*(it*WAVES + w) + l/CPR; with WAVES even the swizzled chunk of its
-// slot, (l % CPR) ^ rswz(r), is the same for every `it`.  Rows past the
-// operand's end reload its last row (their results are never stored).
-template <int ROWS, int NT, int BK>
-struct TileLoad {
-  static constexpr int CPR = BK / 8;    // 16-byte chunks per row
-  static constexpr int RPI = 64 / CPR;  // rows per 1 KB instruction
-  static constexpr int WAVES = NT / 64;
-  static constexpr int ITERS = ROWS / (RPI * WAVES);
-  static_assert(WAVES % 2 == 0 && ITERS * RPI * WAVES == ROWS, "tile/thread mismatch");
-  const char* src[ITERS];  // row base + this lane's chunk, at k = 0
-  int chunk;
-
-  __device__ __forceinline__ void init(const char* base, int64_t ld_bytes, int64_t row0, int64_t rows) {
-    const int lane = threadIdx.x & 63, wave = wave_id();
-    const int r = wave * RPI + lane / CPR;
-    chunk = (lane % CPR) ^ rswz<BK>(r);
-#pragma unroll
-    for (int it = 0; it < ITERS; ++it) {
-      int64_t row = row0 + r + it * RPI * WAVES;
-      if (row > rows - 1) row = rows - 1;
-      src[it] = base + row * ld_bytes + chunk * 16;
-    }
-  }
-  // KT: the K range may end inside this BK slab; a chunk starting past
-  // kend_bytes reloads chunk 0 (masked out of the MFMAs, address valid).
-  template <bool KT>
-  __device__ __forceinline__ void issue(int64_t k0_bytes, char* dst, int64_t kend_bytes) const {
-    const int64_t koff = (KT && k0_bytes + chunk * 16 >= kend_bytes) ? k0_bytes - chunk * 16 : k0_bytes;
-    // one scalar LDS base per call; each instruction's slot is a constant offset
-    const unsigned lds0 = lds_base_of(dst) + wave_id() * 1024;
-#pragma unroll
-    for (int it = 0; it < ITERS; ++it) dma_b128(src[it] + koff, lds0 + it * WAVES * 1024);
-  }
-  template <bool KT>
-  __device__ __forceinline__ void issue_range(int64_t k0_bytes, char* dst, int64_t kend_bytes, int lo, int hi) const {
-    const int64_t koff = (KT && k0_bytes + chunk * 16 >= kend_bytes) ? k0_bytes - chunk * 16 : k0_bytes;
-    const unsigned lds0 = lds_base_of(dst) + wave_id() * 1024;
-#pragma unroll
-    for (int it = 0; it < ITERS; ++it)
-      if (it >= lo && it < hi) dma_b128(src[it] + koff, lds0 + it * WAVES * 1024);
-  }
-};
-
-// m/n-contiguous operand tile: BK k-rows of ROWS elements, 16-byte chunks
-// XOR-swizzled by s(k) = 2 * ((k & 3) | ((k >> 1) & 4)).  A transposing
-// fragment read serves each half-wave from 8 k-rows x 2 adjacent chunks
-// (c, c ^ 1); s takes 8 distinct even values on those k-rows, so the 16
-// (k-row, chunk) pairs land on 16 distinct 16-byte bank groups.
-__device__ __forceinline__ int kswz(int k) { return 2 * ((k & 3) | ((k >> 1) & 4)); }
-
-template <int ROWS, int NT, int BK>
-struct TileLoadT {
-  static constexpr int ROWB = ROWS * 2;
-  static constexpr int CPR = ROWS / 8;     // chunks per k-row
-  static constexpr int KPI = 1024 / ROWB;  // k-rows per 1 KB instruction
-  static constexpr int WAVES = NT / 64;
-  static constexpr int ITERS = BK / KPI / WAVES;
-  static_assert(CPR >= 16 && ITERS * KPI * WAVES == BK, "tile/thread mismatch");
-  const char* base;
-  int64_t ld;              // bytes between k-rows
-  int64_t col_off[ITERS];  // byte offset of this lane's (clamped) chunk
-  int kr[ITERS];           // this lane's k-row within the slab
-
-  // A last partial chunk of rows reads into the row padding (the k stride
-  // is at least the row count rounded up to 8, checked by the caller).
-  __device__ __forceinline__ void init(const char* b, int64_t ld_bytes, int64_t r0, int64_t rows) {
-    const int lane = threadIdx.x & 63, wave = wave_id();
-    base = b;
-    ld = ld_bytes;
-    const int64_t last_chunk = ((rows - 1) >> 3) << 3;
-#pragma unroll
-    for (int it = 0; it < ITERS; ++it) {
-      kr[it] = (it * WAVES + wave) * KPI + lane / CPR;
-      int64_t m = r0 + ((lane % CPR) ^ kswz(kr[it])) * 8;
-      if (m > last_chunk) m = last_chunk;
-      col_off[it] = m * 2;
-    }
-  }
-  // KT: k-rows at or past kend reload row kend-1 (masked out of the MFMAs).
-  template <bool KT>
-  __device__ __forceinline__ void issue(int64_t k0, char* dst, int64_t kend) const {
-    const unsigned lds0 = lds_base_of(dst) + wave_id() * 1024;
-#pragma unroll
-    for (int it = 0; it < ITERS; ++it) {
-      int64_t k = k0 + kr[it];
-      if (KT && k >= kend) k = kend - 1;
-      dma_b128(base + k * ld + col_off[it], lds0 + it * WAVES * 1024);
-    }
-  }
-  template <bool KT>
-  __device__ __forceinline__ void issue_range(int64_t k0, char* dst, int64_t kend, int lo, int hi) const {
-    const unsigned lds0 = lds_base_of(dst) + wave_id() * 1024;
-#pragma unroll
-    for (int it = 0; it < ITERS; ++it) {
-      if (it < lo || it >= hi) continue;
-      int64_t k = k0 + kr[it];
-      if (KT && k >= kend) k = kend - 1;
-      dma_b128(base + k * ld + col_off[it], lds0 + it * WAVES * 1024);
-    }
-  }
-};
-
-template <int ROWS, int NT, bool K_CONTIG, int BK>
-struct OperandLoad;
-template <int ROWS, int NT, int BK>
-struct OperandLoad<ROWS, NT, true, BK> {
-  TileLoad<ROWS, NT, BK> t;
-  __device__ __forceinline__ void init(const char* b, int64_t ld, int64_t r0, int64_t n) { t.init(b, ld, r0, n); }
-  template <bool KT>
-  __device__ __forceinline__ void issue(int64_t k0, char* dst, int64_t kend) const {
-    t.template issue<KT>(k0 * 2, dst, kend * 2);
-  }
-  template <bool KT>
-  __device__ __forceinline__ void issue_range(int64_t k0, char* dst, int64_t kend, int lo, int hi) const {
-    t.template issue_range<KT>(k0 * 2, dst, kend * 2, lo, hi);
-  }
-  static constexpr int ITERS = TileLoad<ROWS, NT, BK>::ITERS;
-};
-template <int ROWS, int NT, int BK>
-struct OperandLoad<ROWS, NT, false, BK> {
-  TileLoadT<ROWS, NT, BK> t;
-  __device__ __forceinline__ void init(const char* b, int64_t ld, int64_t r0, int64_t n) { t.init(b, ld, r0, n); }
-  template <bool KT>
-  __device__ __forceinline__ void issue(int64_t k0, char* dst, int64_t kend) const {
-    t.template issue<KT>(k0, dst, kend);
-  }
-  template <bool KT>
-  __device__ __forceinline__ void issue_range(int64_t k0, char* dst, int64_t kend, int lo, int hi) const {
-    t.template issue_range<KT>(k0, dst, kend, lo, hi);
-  }
-  static constexpr int ITERS = TileLoadT<ROWS, NT, BK>::ITERS;
-};
-
-
-// CNT MFMA fragments (rows r0 + 16i .. +15, k = ks*32 + 8g + 0..7) from an
-// m/n-contiguous tile, two transposing reads each: within a 16-lane group,
-// lane i receives element i%4 of the 4-element pieces of lanes i/4, 4+i/4,
-// 8+i/4, 12+i/4, so source lane 4e+q supplies k-row (.. + e), columns
-// r0+4q..+3.
-template <typename T, int ROWS, int CNT>
-__device__ __forceinline__ void mn_frags(const char* tile, int r0, int ks, typename Mfma<T>::frag (&f)[CNT]) {
-  constexpr int ROWB = ROWS * 2;
-  const int lane = threadIdx.x & 63;
-  const int g = lane >> 4, src = lane & 15;
-  const int k1 = ks * 32 + 8 * g + (src >> 2), k2 = k1 + 4;
-#pragma unroll
-  for (int i = 0; i < CNT; ++i) {
-    const int m = r0 + i * 16 + 4 * (src & 3);
-    const s16x4 a = ds_read_tr(tile + k1 * ROWB + (((m >> 3) ^ kswz(k1)) << 4) + ((m & 7) << 1));
-    const s16x4 b = ds_read_tr(tile + k2 * ROWB + (((m >> 3) ^ kswz(k2)) << 4) + ((m & 7) << 1));
-    f[i] = join_frag<typename Mfma<T>::frag>(a, b);
-  }
-}
-
-// Zero the fragment slots whose k index (kbase + slot) is >= kend.
-template <typename F>
-__device__ __forceinline__ void mask_k(F& f, int64_t kbase, int64_t kend) {
-  short* fs = (short*)&f;
-#pragma unroll
-  for (int e = 0; e < 8; ++e)
-    if (kbase + e >= kend) fs[e] = 0;
-}
-
-// Block configurations.
-#ifndef GEMM_STAGES_128
-#define GEMM_STAGES_128 2
-#endif
-#ifndef GEMM_STAGES_192
-#define GEMM_STAGES_192 2
-#endif
-template <int CFG>
-struct TileCfg;
-template <>
-struct TileCfg<0> {  // C128
-  static constexpr int BM = 128, BN = 128, BK = 64, WGM = 2, WGN = 2, STAGES = GEMM_STAGES_128;
-  static constexpr int MIN_BLOCKS = STAGES * (BM + BN) * BK * 2 * 2 <= 160 * 1024 ? 2 : 1;
-};
-template <>
-struct TileCfg<1> {  // C256
-  static constexpr int BM = 256, BN = 256, BK = 64, WGM = 2, WGN = 4, STAGES = 2, MIN_BLOCKS = 1;
-};
-template <>
-struct TileCfg<2> {  // C192: 128x192, waves of 64x96, 40 KB per stage (k-contiguous B only)
-  static constexpr int BM = 128, BN = 192, BK = 64, WGM = 2, WGN = 2, STAGES = GEMM_STAGES_192;
-  static constexpr int MIN_BLOCKS = STAGES * (BM + BN) * BK * 2 * 2 <= 160 * 1024 ? 2 : 1;
-};
-// C256 in 32-k stages, three deep (96 KB): for weight gradients, whose
-// operands are both m/n-contiguous.  Their transposing fragment reads make
-// a 64-k step long; halving it and keeping two stages in flight hides the
-// loads better (gfx950, cfg 2 shapes: 7-13% over 64-k stages).
-template <>
-struct TileCfg<3> {
-  static constexpr int BM = 256, BN = 256, BK = 32, WGM = 2, WGN = 4, STAGES = 3, MIN_BLOCKS = 1;
-};
-
-// s_waitcnt immediate for vmcnt(n), other counters not waited on.
-constexpr int vmcnt_imm(int n) { return 0x0f70 | (n & 15) | ((n >> 4) << 14); }
-
-// Write one wave's accumulators to C (pointing at the wave tile's first
-// element), adding the preloaded bias and, with BETA, the old C.  Offsets
-// inside the tile are 32-bit (the host checks the row stride); EDGE adds the
-// bounds checks that only partial tiles need.  Each store instruction covers
-// four 16-column runs, and the j loop fills whole 128-byte lines.
-template <typename CT, typename T, bool BETA, bool EDGE, bool ROUND, int TM, int TN>
-__device__ __forceinline__ void store_tile(CT* __restrict__ C, int c_rs, const f32x4 (&acc)[TM][TN],
-                                           const float (&bias)[TN], int rows_left, int cols_left, int lr,
-                                           int lg) {
-#pragma unroll
-  for (int i = 0; i < TM; ++i)
-#pragma unroll
-    for (int e = 0; e < 4; ++e) {
-      const int r = i * 16 + lg * 4 + e;
-      if (EDGE && r >= rows_left) continue;
-      CT* row = C + r * c_rs;
-#pragma unroll
-      for (int j = 0; j < TN; ++j) {
-        const int c = j * 16 + lr;
-        if (EDGE && c >= cols_left) continue;
-        float v = acc[i][j][e] + bias[j];
-        if (BETA) v += (float)row[c];
-        if (ROUND) v = (float)(T)v;
-        row[c] = (CT)v;
-      }
-    }
-}
-
-// Full wave tiles without beta: the accumulators go through a per-wave LDS
-// slab 16 rows at a time (one MFMA row of tiles, f32, rows padded by 4
-// floats) and leave as row-contiguous 16-byte stores: 8 bf16/f16 or 4 f32
-// per lane instead of one element per store.  The slab holds 16 x (WN + 4)
-// floats; `lane` is the wave lane.  Requires 16-byte aligned rows of C.
-// NT: non-temporal stores, for outputs no kernel reads soon enough to find
-// them in a cache (split-K partials, summed right after, keep normal
-// stores); a training step ran 0.2 ms faster with them.
-template <typename CT, typename T, bool ROUND, bool NT, int TM, int TN>
-__device__ __forceinline__ void store_tile_lds(CT* __restrict__ C, int c_rs, const f32x4 (&acc)[TM][TN],
-                                               const float (&bias)[TN], float* slab, int lr, int lg, int lane) {
-#ifndef GEMM_SLAB_PAD
-#define GEMM_SLAB_PAD 4
-#endif
-  // slab row stride in floats: 4 * LD = 16 (mod 64) puts the four 16-lane
-  // groups of a store (rows lg*4 + e) on disjoint banks
-  constexpr int WN = TN * 16, LD = WN + GEMM_SLAB_PAD;
-  constexpr int E = 16 / sizeof(CT);             // elements per 16-byte store
-  constexpr int CHUNKS = 16 * WN / E;            // 16-byte chunks per 16-row slab
-  static_assert(WN % E == 0 && CHUNKS % 64 == 0, "slab shape");
-#pragma unroll
-  for (int i = 0; i < TM; ++i) {
-#pragma unroll
-    for (int j = 0; j < TN; ++j)
-#pragma unroll
-      for (int e = 0; e < 4; ++e) {
-        float v = acc[i][j][e] + bias[j];
-        if (ROUND) v = (float)(T)v;
-        slab[(lg * 4 + e) * LD + j * 16 + lr] = v;
-      }
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-    __builtin_amdgcn_wave_barrier();
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-#pragma unroll
-    for (int it = 0; it < CHUNKS / 64; ++it) {
-      const int ch = it * 64 + lane, r = ch / (WN / E), c = (ch % (WN / E)) * E;
-      const float* src = slab + r * LD + c;
-      struct alignas(16) Out { CT v[E]; } out;
-#pragma unroll
-      for (int e = 0; e < E; ++e) out.v[e] = (CT)src[e];
-      if constexpr (NT)
-        __builtin_nontemporal_store(__builtin_bit_cast(f32x4, out), (f32x4*)(C + (i * 16 + r) * c_rs + c));
-      else
-        *(Out*)(C + (i * 16 + r) * c_rs + c) = out;
-    }
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-    __builtin_amdgcn_wave_barrier();
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-  }
-}
-
-template <typename CT, typename T, int TM, int TN>
-__device__ __forceinline__ void store_any(CT* C, int c_rs, const f32x4 (&acc)[TM][TN], const float (&bias)[TN],
-                                          bool beta, bool round, int rows_left, int cols_left, int lr, int lg) {
-  const bool edge = rows_left < TM * 16 || cols_left < TN * 16;
-#define ST(B, E, R) store_tile<CT, T, B, E, R>(C, c_rs, acc, bias, rows_left, cols_left, lr, lg)
-  if (round) {  // round-through stores are only used without beta
-    if (edge) ST(false, true, true);
-    else ST(false, false, true);
-  } else if (beta) {
-    if (edge) ST(true, true, false);
-    else ST(true, false, false);
-  } else {
-    if (edge) ST(false, true, false);
-    else ST(false, false, false);
-  }
-#undef ST
-}
-
-// RS: also sum A's rows over k, from the fragments the MFMAs consume, with
-// one extra MFMA against a fragment of ones (every column of its 16x16
-// result is the row sum).  With split K the 32-k substeps are dealt round
-// robin over the tiles_n * WGN waves that hold the same rows (one substep in
-// that many per wave), each writing its own partial slot; without split K
-// the waves of the first wave column of the first column tile do it all.
-template <typename T, int CFG, bool A_K, bool B_K, bool KT, bool RS>
-__global__ void __launch_bounds__(64 * TileCfg<CFG>::WGM * TileCfg<CFG>::WGN, TileCfg<CFG>::MIN_BLOCKS)
-    gemm_tile(GemmArgs g) {
-  typedef typename Mfma<T>::frag frag;
-  typedef TileCfg<CFG> C;
-  constexpr int BM = C::BM, BN = C::BN;
-  constexpr int NT = 64 * C::WGM * C::WGN;
-  constexpr int WM = BM / C::WGM, WN = BN / C::WGN;
-  constexpr int TM = WM / 16, TN = WN / 16;
-  constexpr int BK = C::BK, ROWB = BK * 2;  // k per stage, bytes of a k-contiguous row
-  constexpr int A_BYTES = BM * ROWB, STAGE = A_BYTES + BN * ROWB, S = C::STAGES;
-  char* const lds = gemm_smem;
-
-#if GEMM_XCD_FLAT
-  // XCD-aware order over the whole grid: the hardware deals workgroups to
-  // the 8 XCDs round-robin in dispatch order (x fastest, then y), so XCD
-  // L % 8 gets every 8th block.  Each XCD is given one contiguous run of the
-  // (split, batch)-major tile list instead: its blocks share A/B panels and,
-  // with split K, one or two K ranges, so each L2 fetches about 1/8 of the
-  // operands (dealing a plane's tiles over all XCDs made every L2 fetch
-  // every split's panels).  A bijection for any grid size.
-  const uint32_t nt = gridDim.x;
-  uint32_t L = blockIdx.x + nt * blockIdx.y;
-  {
-    const uint32_t total = nt * gridDim.y, xcd = L & 7, q = total >> 3, r = total & 7;
-    L = xcd * q + min(xcd, r) + (L >> 3);
-  }
-  const uint32_t plane = L / nt, t = L - plane * nt;
-  const uint32_t tm = t / (uint32_t)g.tiles_n, tn = t - tm * (uint32_t)g.tiles_n;
-  const uint32_t split = plane / (uint32_t)g.batch, bidx = plane - split * (uint32_t)g.batch;
-#else
-  // XCD-aware tile order within one (split, batch) plane.
-  uint32_t t = blockIdx.x;
-  const uint32_t nt = gridDim.x;
-  if ((nt & 7) == 0) t = (t & 7) * (nt >> 3) + (t >> 3);
-  const uint32_t tm = t / (uint32_t)g.tiles_n, tn = t - tm * (uint32_t)g.tiles_n;
-  const uint32_t split = blockIdx.y / (uint32_t)g.batch, bidx = blockIdx.y - split * (uint32_t)g.batch;
-#endif
-  const int64_t m0 = (int64_t)tm * BM, n0 = (int64_t)tn * BN;
-  int64_t kbeg = 0, kend = g.k;
-  if (g.part) {
-    kbeg = (int64_t)split * g.kchunk;
-    kend = min(g.k, kbeg + g.kchunk);
-  }
-
-  const char* A = (const char*)g.a + (int64_t)bidx * g.a_bs * (int64_t)sizeof(T);
-  const char* B = (const char*)g.b + (int64_t)bidx * g.b_bs * (int64_t)sizeof(T);
-  // A_K: bytes between rows; else bytes between k-rows.  Same for B.
-  const int64_t a_ldb = (A_K ? g.a_rs : g.a_cs) * (int64_t)sizeof(T);
-  const int64_t b_ldb = (B_K ? g.b_cs : g.b_rs) * (int64_t)sizeof(T);
-
-  const int lane = threadIdx.x & 63, wave = wave_id();  // scalar: the row-sum test branches on it
-  const int wm = wave / C::WGN, wn = wave % C::WGN;
-  const int lr = lane & 15, lg = lane >> 4;
-
-  f32x4 acc[TM][TN];
-#pragma unroll
-  for (int i = 0; i < TM; ++i)
-#pragma unroll
-    for (int j = 0; j < TN; ++j) acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
-
-  OperandLoad<BM, NT, A_K, BK> la;
-  OperandLoad<BN, NT, B_K, BK> lb;
-  constexpr int PER_STAGE = decltype(la.t)::ITERS + decltype(lb.t)::ITERS;  // DMA instructions per stage
-  static_assert(S == 2 || (S - 2) * PER_STAGE < 64, "vmcnt range");
-  la.init(A, a_ldb, m0, g.m);
-  lb.init(B, b_ldb, n0, g.n);
-  // Prologue: stages 0 .. S-2 in flight.
-#pragma unroll
-  for (int st = 0; st < S - 1; ++st) {
-    if (kbeg + st * BK < kend) {
-      la.template issue<KT>(kbeg + st * BK, lds + st * STAGE, kend);
-      lb.template issue<KT>(kbeg + st * BK, lds + st * STAGE + A_BYTES, kend);
-    }
-  }
-  // k-contiguous fragment rows (.. + lr) share the swizzle of lr
-  const int sw = rswz<BK>(lr);
-  const int rs_slots = g.part ? g.tiles_n * C::WGN : 1;
-  const int rs_slot = g.part ? (int)tn * C::WGN + wn : 0;
-  const bool rs_on = RS && (g.part || (tn == 0 && wn == 0));
-  int rs_q = 0;  // this wave's substep counter modulo rs_slots
-  f32x4 rsum[TM];
-  frag ones;
-#pragma unroll
-  for (int i = 0; i < TM; ++i) rsum[i] = f32x4{0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-  for (int e = 0; e < 8; ++e) ones[e] = (T)1.0f;
-
-  int cur = 0;
-  for (int64_t k0 = kbeg; k0 < kend; k0 += BK) {
-    // This step's tiles have landed when at most the later stages' loads
-    // (S-2 stages, if issued) are still outstanding.
-    if (S > 2 && k0 + (S - 2) * BK < kend) __builtin_amdgcn_s_waitcnt(vmcnt_imm((S - 2) * PER_STAGE));
-    else __builtin_amdgcn_s_waitcnt(vmcnt_imm(0));
-    __syncthreads();
-    // the next stage goes to the slot read in the previous step (every wave
-    // is past it); its loads are issued after this step's first B fragment
-    // reads, so the first MFMAs do not wait behind the load issue (training
-    // step 22.22 -> 22.03 ms, three runs each on one box; issuing them after
-    // the reads only for k-contiguous A gave nothing).  The 256x256 tiles
-    // (eight MFMA rows per wave) spread the load instructions over the MFMA
-    // rows of the first 32-k substep instead, so the load issue no longer
-    // stalls the wave in one burst: the forward fc and lm_head launches run
-    // 3.4-5.8% faster in the training step (kernel trace, two boxes); the
-    // same spread lost 2-6% on the 128x128 and 128x192 tiles and the 32-k
-    // 256x256 weight-gradient tiles, which keep the single burst.
-    const bool more = k0 + (S - 1) * BK < kend;
-    char* const nxt = lds + (cur == 0 ? S - 1 : cur - 1) * STAGE;
-    const char* at = lds + cur * STAGE;
-    const char* bt = at + A_BYTES;
-    const bool tail = KT && k0 + BK > kend;
-#pragma unroll
-    for (int ks = 0; ks < BK / 32; ++ks) {
-      const bool rs_now = rs_on && rs_q == rs_slot;
-      if (RS && ++rs_q == rs_slots) rs_q = 0;
-      const int coff = ((ks * 4 + lg) ^ sw) * 16;
-      const int64_t kfrag = k0 + ks * 32 + lg * 8;
-      frag bfr[TN], afr[A_K ? 1 : TM];
-      if constexpr (!B_K) mn_frags<T, BN, TN>(bt, wn * WN, ks, bfr);
-      if constexpr (!A_K) mn_frags<T, BM, TM>(at, wm * WM, ks, afr);
-#pragma unroll
-      for (int j = 0; j < TN; ++j) {
-        if constexpr (B_K) bfr[j] = *(const frag*)(bt + (wn * WN + j * 16 + lr) * ROWB + coff);
-        if (tail) mask_k(bfr[j], kfrag, kend);
-      }
-      if (CFG != 1 && ks == 0 && more) {
-        la.template issue<KT>(k0 + (S - 1) * BK, nxt, kend);
-        lb.template issue<KT>(k0 + (S - 1) * BK, nxt + A_BYTES, kend);
-      }
-#pragma unroll
-      for (int i = 0; i < TM; ++i) {
-        if (CFG == 1 && ks == 0 && more) {
-          // load instructions q in [lo, hi) of this stage's list (A's, then B's)
-          constexpr int NA = decltype(la)::ITERS, NQ = NA + decltype(lb)::ITERS;
-          const int lo = i * NQ / TM, hi = (i + 1) * NQ / TM;
-          la.template issue_range<KT>(k0 + (S - 1) * BK, nxt, kend, lo, hi);
-          lb.template issue_range<KT>(k0 + (S - 1) * BK, nxt + A_BYTES, kend, lo - NA, hi - NA);
-        }
-        frag af;
-        if constexpr (A_K) af = *(const frag*)(at + (wm * WM + i * 16 + lr) * ROWB + coff);
-        else af = afr[i];
-        if (tail) mask_k(af, kfrag, kend);
-        if (RS && rs_now) rsum[i] = Mfma<T>::mma(af, ones, rsum[i]);
-#pragma unroll
-        for (int j = 0; j < TN; ++j) acc[i][j] = Mfma<T>::mma(af, bfr[j], acc[i][j]);
-      }
-    }
-    cur = cur == S - 1 ? 0 : cur + 1;
-  }
-
-  // every wave is past its last LDS read: the stages become store slabs
-  __syncthreads();
-  float* const slab = (float*)lds + wave * (16 * (WN + GEMM_SLAB_PAD));
-  const int64_t row0 = m0 + wm * WM, col0 = n0 + wn * WN;
-  if (RS && rs_on && lr == 0) {
-    // lane (lg, 0) holds rows 4*lg .. 4*lg+3 of each 16-row fragment
-    const int64_t slot = (int64_t)split * rs_slots + rs_slot;
-#pragma unroll
-    for (int i = 0; i < TM; ++i)
-#pragma unroll
-      for (int e = 0; e < 4; ++e) {
-        const int64_t r = row0 + i * 16 + lg * 4 + e;
-        if (r >= g.m) continue;
-        if (g.part) {
-          g.rs_part[(slot * g.batch + bidx) * g.m + r] = rsum[i][e];
-        } else {
-          const float v = g.round_c ? round_through(rsum[i][e], g.ab_dt) : rsum[i][e];
-          st_any(g.rowsum, g.rowsum_dt, (int64_t)bidx * g.m + r, v);
-        }
-      }
-  }
-  const int rows_left = (int)min(g.m - row0, (int64_t)WM), cols_left = (int)min(g.n - col0, (int64_t)WN);
-  if (rows_left <= 0 || cols_left <= 0) return;
-  float bias[TN];
-  if (g.part) {
-#pragma unroll
-    for (int j = 0; j < TN; ++j) bias[j] = 0.f;
-    float* P = g.part + ((int64_t)split * g.batch + bidx) * g.m * g.n + row0 * g.n + col0;
-    if (rows_left == WM && cols_left == WN && (g.n & 3) == 0 && ((uintptr_t)g.part & 15) == 0)
-      store_tile_lds<float, T, false, false>(P, (int)g.n, acc, bias, slab, lr, lg, lane);
-    else
-      store_any<float, T>(P, (int)g.n, acc, bias, false, false, rows_left, cols_left, lr, lg);
-    return;
-  }
-#pragma unroll
-  for (int j = 0; j < TN; ++j) {
-    const int c = j * 16 + lr;
-    bias[j] = (g.bias && c < cols_left) ? ld_any(g.bias, g.bias_dt, col0 + c) : 0.f;
-  }
-  const int64_t c_es = g.c_dt == MI355X_F32 ? 4 : 2;
-  char* Cb = (char*)g.c + ((int64_t)bidx * g.c_bs + row0 * g.c_rs + col0) * c_es;
-  const int c_rs = (int)g.c_rs;
-  const bool rnd = g.round_c && g.c_dt == MI355X_F32;  // 16-bit outputs are already rounded
-  const bool full = rows_left == WM && cols_left == WN && !g.beta && ((uintptr_t)g.c & 15) == 0 &&
-                    (c_rs * c_es) % 16 == 0 && (g.c_bs * c_es) % 16 == 0;
-  if (full) {
-    if (g.c_dt == MI355X_BF16) store_tile_lds<bf16, T, false, true>((bf16*)Cb, c_rs, acc, bias, slab, lr, lg, lane);
-    else if (g.c_dt == MI355X_F16) store_tile_lds<f16, T, false, true>((f16*)Cb, c_rs, acc, bias, slab, lr, lg, lane);
-    else if (rnd) store_tile_lds<float, T, true, true>((float*)Cb, c_rs, acc, bias, slab, lr, lg, lane);
-    else store_tile_lds<float, T, false, true>((float*)Cb, c_rs, acc, bias, slab, lr, lg, lane);
-    return;
-  }
-  if (g.c_dt == MI355X_BF16) store_any<bf16, T>((bf16*)Cb, c_rs, acc, bias, g.beta, false, rows_left, cols_left, lr, lg);
-  else if (g.c_dt == MI355X_F32) store_any<float, T>((float*)Cb, c_rs, acc, bias, g.beta, rnd, rows_left, cols_left, lr, lg);
-  else store_any<f16, T>((f16*)Cb, c_rs, acc, bias, g.beta, false, rows_left, cols_left, lr, lg);
-}
-
 // Pack an operand into a k-contiguous [rows][ld] buffer of 16-bit elements,
 // zero-filling k in [K, ld).  Source element (row, k) is at
 //   transposed: src + b*sbs + k*sk + row      (row-contiguous source)
@@ -779,17 +223,28 @@ struct Plan {
   int64_t kchunk;
 };
 
+// Rows and columns of C per block, and the waves along them.
+struct CfgShape {
+  int bm, bn, wgn;
+};
+CfgShape shape_of(int cfg) {
+  switch (cfg) {
+    case 1: case 3: return {256, 256, 4};
+    case 2: return {128, 192, 2};
+    case 4: return {64, 64, 2};
+    default: return {128, 128, 2};
+  }
+}
+
 int64_t tiles_of(int cfg, int64_t batch, int64_t m, int64_t n) {
-  const bool c256 = cfg == 1 || cfg == 3;
-  const int64_t bm = c256 ? 256 : 128, bn = c256 ? 256 : (cfg == 2 ? 192 : 128);
-  return ((m + bm - 1) / bm) * ((n + bn - 1) / bn) * batch;
+  const CfgShape c = shape_of(cfg);
+  return ((m + c.bm - 1) / c.bm) * ((n + c.bn - 1) / c.bn) * batch;
 }
 
 // Row-sum partial slots per split: one per wave column of every column tile.
 int64_t rs_slots_of(int cfg, int64_t n) {
-  const bool c256 = cfg == 1 || cfg == 3;
-  const int64_t bn = c256 ? 256 : (cfg == 2 ? 192 : 128), wgn = c256 ? 4 : 2;
-  return (n + bn - 1) / bn * wgn;
+  const CfgShape c = shape_of(cfg);
+  return (n + c.bn - 1) / c.bn * c.wgn;
 }
 
 // Pick the configuration that finishes in the least time: whole rounds of
@@ -816,10 +271,19 @@ Plan plan_gemm(int64_t batch, int64_t m, int64_t n, int64_t k, bool a_kcontig, b
   // L2s (config 2 shapes, TF/s: 768 x 768 646 against 501, 2304 x 768 912
   // against 839, 768 x 3072 933 against 915).
   if (!a_kcontig && m >= 256 && n >= 256 && t256 >= kCUs) best.cfg = 3;
+  // Outputs of at most two 64x64 tiles per CU: their larger tiles leave CUs
+  // idle and a k-step takes its latencies, not its MFMA time (us, larger
+  // tiles against C64; K = 768 unless given: 77 x 768 11.6 / 6.3, 255 x 2304
+  // 18.1 / 7.5, 512 x 3072 10.9 / 9.6, 1021 x 1024 at K = 1152 20.6 / 9.3,
+  // 2048 x 768 10.8 / 7.9; weight gradients 768 x 768 at K = 4096 22.7 / 17.0,
+  // 2304 x 768 at K = 2048 24.3 / 15.6).  Past that the larger tiles win
+  // (768 tiles, 4096 x 768: 11.4 / 12.7; 576, 768 x 3072 at K = 2048:
+  // 24.5 / 26.4).
+  if (tiles_of(4, batch, m, n) <= 2 * kCUs) best.cfg = 4;
   static const char* forced = getenv("MI355X_GEMM_TILE");  // tuning override: "128", "192", "256" or "256.32"
   if (forced) {
     const double f = atof(forced);
-    best.cfg = f == 256 ? 1 : (f > 256 && !a_kcontig ? 3 : (f == 192 && b_kcontig ? 2 : 0));
+    best.cfg = f == 256 ? 1 : (f > 256 && !a_kcontig ? 3 : (f == 192 && b_kcontig ? 2 : (f == 64 ? 4 : 0)));
   }
   const int64_t tiles = tiles_of(best.cfg, batch, m, n);
   if (best.cfg == 3 && tiles >= kCUs && k >= 8192) {
@@ -858,54 +322,6 @@ Plan plan_gemm(int64_t batch, int64_t m, int64_t n, int64_t k, bool a_kcontig, b
     }
   }
   return best;
-}
-
-// Launch one kernel instantiation; the first launch of each opts it into
-// more than 64 KB of dynamic LDS when it needs that.
-template <typename T, int CFG, bool A_K, bool B_K, bool KT, bool RS>
-int launch_kernel(const GemmArgs& g, dim3 grid, hipStream_t s) {
-  typedef TileCfg<CFG> C;
-  constexpr int NT = 64 * C::WGM * C::WGN;
-  constexpr size_t lds = C::STAGES * (size_t)(C::BM + C::BN) * C::BK * 2;
-  static bool attr = false;
-  if (lds > 65536 && !attr) {
-    if (hipFuncSetAttribute((const void*)gemm_tile<T, CFG, A_K, B_K, KT, RS>,
-                            hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds) != hipSuccess)
-      return fail(MI355X_ELAUNCH, "mi355x_gemm: cannot reserve %zu bytes of LDS", lds);
-    attr = true;
-  }
-  gemm_tile<T, CFG, A_K, B_K, KT, RS><<<grid, NT, lds, s>>>(g);
-  return check_launch("mi355x_gemm");
-}
-
-template <typename T, int CFG, bool KT, bool RS>
-int launch_layout(const GemmArgs& g, dim3 grid, hipStream_t s) {
-  const bool ak = g.a_cs == 1, bk = g.b_rs == 1;
-  if constexpr (CFG == 3) {  // chosen for m-contiguous A only
-    if (ak) return fail(MI355X_EINVAL, "mi355x_gemm: 32-k C256 tiles take an m-contiguous A");
-    if (bk) return launch_kernel<T, CFG, false, true, KT, RS>(g, grid, s);
-    return launch_kernel<T, CFG, false, false, KT, RS>(g, grid, s);
-  } else if constexpr (CFG == 2) {  // 192-wide B tiles are only loaded k-contiguous
-    if (!bk) return fail(MI355X_EINVAL, "mi355x_gemm: 128x192 tiles need a k-contiguous B");
-    if (ak) return launch_kernel<T, CFG, true, true, KT, RS>(g, grid, s);
-    return launch_kernel<T, CFG, false, true, KT, RS>(g, grid, s);
-  } else {
-    if (ak && bk) return launch_kernel<T, CFG, true, true, KT, RS>(g, grid, s);
-    if (ak) return launch_kernel<T, CFG, true, false, KT, RS>(g, grid, s);
-    if (bk) return launch_kernel<T, CFG, false, true, KT, RS>(g, grid, s);
-    return launch_kernel<T, CFG, false, false, KT, RS>(g, grid, s);
-  }
-}
-
-template <typename T, int CFG, bool KT>
-int launch_tile(GemmArgs g, int64_t batch, int splits, hipStream_t s) {
-  typedef TileCfg<CFG> C;
-  const int tm = (int)ceil_div(g.m, C::BM), tn = (int)ceil_div(g.n, C::BN);
-  g.tiles_n = tn;
-  g.batch = (int)batch;
-  dim3 grid((unsigned)(tm * tn), (unsigned)(batch * splits));
-  if (g.rowsum) return launch_layout<T, CFG, KT, true>(g, grid, s);
-  return launch_layout<T, CFG, KT, false>(g, grid, s);
 }
 
 }  // namespace
@@ -949,11 +365,7 @@ namespace {
 template <typename T>
 int launch_mfma(GemmArgs g, int64_t batch, const Plan& p, hipStream_t s) {
   const bool kt = g.k % 64 != 0;
-  int rc;
-  if (p.cfg == 1) rc = kt ? launch_tile<T, 1, true>(g, batch, p.splits, s) : launch_tile<T, 1, false>(g, batch, p.splits, s);
-  else if (p.cfg == 3) rc = kt ? launch_tile<T, 3, true>(g, batch, p.splits, s) : launch_tile<T, 3, false>(g, batch, p.splits, s);
-  else if (p.cfg == 2) rc = kt ? launch_tile<T, 2, true>(g, batch, p.splits, s) : launch_tile<T, 2, false>(g, batch, p.splits, s);
-  else rc = kt ? launch_tile<T, 0, true>(g, batch, p.splits, s) : launch_tile<T, 0, false>(g, batch, p.splits, s);
+  int rc = kt ? gemm_tiles<T, true>(g, batch, p.cfg, p.splits, s) : gemm_tiles<T, false>(g, batch, p.cfg, p.splits, s);
   if (rc || !g.part) return rc;
   const int rs_slots = g.rowsum ? (int)(p.splits * rs_slots_of(p.cfg, g.n)) : 0;
   rc = splitk_finish(g, batch, p.splits, rs_slots, s);
