@@ -271,15 +271,17 @@ Plan plan_gemm(int64_t batch, int64_t m, int64_t n, int64_t k, bool a_kcontig, b
   // L2s (config 2 shapes, TF/s: 768 x 768 646 against 501, 2304 x 768 912
   // against 839, 768 x 3072 933 against 915).
   if (!a_kcontig && m >= 256 && n >= 256 && t256 >= kCUs) best.cfg = 3;
-  // Outputs of at most two 64x64 tiles per CU: their larger tiles leave CUs
-  // idle and a k-step takes its latencies, not its MFMA time (us, larger
-  // tiles against C64; K = 768 unless given: 77 x 768 11.6 / 6.3, 255 x 2304
-  // 18.1 / 7.5, 512 x 3072 10.9 / 9.6, 1021 x 1024 at K = 1152 20.6 / 9.3,
-  // 2048 x 768 10.8 / 7.9; weight gradients 768 x 768 at K = 4096 22.7 / 17.0,
-  // 2304 x 768 at K = 2048 24.3 / 15.6).  Past that the larger tiles win
-  // (768 tiles, 4096 x 768: 11.4 / 12.7; 576, 768 x 3072 at K = 2048:
-  // 24.5 / 26.4).
-  if (tiles_of(4, batch, m, n) <= 2 * kCUs) best.cfg = 4;
+  // Outputs of at most two 64x64 tiles per CU with up to 5e9 multiply-adds:
+  // their larger tiles leave CUs idle and a k-step takes its latencies, not
+  // its MFMA time (us, larger tiles against C64; K = 768 unless given: 77 x
+  // 768 11.6 / 6.3, 255 x 2304 18.1 / 7.5, 512 x 3072 10.9 / 9.6, 1021 x 1024
+  // at K = 1152 20.6 / 9.3, 2048 x 768 10.8 / 7.9; weight gradients 768 x 768
+  // at K = 4096 22.7 / 17.0, 2304 x 768 at K = 2048 24.3 / 15.6).  Past that
+  // the larger tiles win: more tiles (4096 x 768 11.4 / 12.7, 768 x 3072 at
+  // K = 2048 24.5 / 26.4), or a K long enough to split over all CUs (768 x
+  // 768 at K = 8192 24.2 / 24.2, at 16384 33.4 / 40.9; 1024 x 768 at K = 8192
+  // 26.4 / 29.6).
+  if (tiles_of(4, batch, m, n) <= 2 * kCUs && (double)(batch * m * n) * (double)k <= 5e9) best.cfg = 4;
   static const char* forced = getenv("MI355X_GEMM_TILE");  // tuning override: "128", "192", "256" or "256.32"
   if (forced) {
     const double f = atof(forced);
