@@ -15,6 +15,7 @@ import os
 import shutil
 import subprocess
 import sys
+import sysconfig
 from concurrent.futures import ThreadPoolExecutor
 from pathlib import Path
 
@@ -25,6 +26,9 @@ OBJ_DIR = PKG_DIR / "_build"
 INCLUDE = REPO / "include"
 LIB_NAME = "libmi355x_kernels.so"
 LIB_PATH = PKG_DIR / "torch_mojo_backend" / "eager_kernels" / LIB_NAME
+# the host path (csrc/host): a CPython extension that calls the library
+HOST_SRC = CSRC / "host" / "host.cpp"
+HOST_PATH = PKG_DIR / "torch_mojo_backend" / "eager_kernels" / "_host.so"
 
 ARCH = "gfx950"
 # -packed-fp32-ops: keep the compiler from emitting packed f32 VALU ops.
@@ -83,15 +87,29 @@ def _compile(src: Path, force: bool, defines: tuple[str, ...] = ()) -> Path:
     return obj
 
 
+def _build_host(digest: tuple[str, ...]) -> None:
+    """Compile the host extension (host code only, against this Python)."""
+    tmp = HOST_PATH.with_suffix(".so.tmp")
+    cmd = [shutil.which("g++") or "g++", "-O2", "-std=c++17", "-fPIC", "-shared", *digest,
+           f"-I{sysconfig.get_paths()['include']}", str(HOST_SRC), "-o", str(tmp)]
+    proc = subprocess.run(cmd, capture_output=True, text=True)
+    if proc.returncode != 0:
+        raise RuntimeError(f"compiling {HOST_SRC.name} failed:\n{proc.stderr}")
+    os.replace(tmp, HOST_PATH)
+
+
 def build(force: bool = True, jobs: int | None = None) -> Path:
-    """Compile every csrc/*.hip for gfx950 and link the shared library."""
+    """Compile every csrc/*.hip for gfx950 and link the shared library, and
+    compile the host extension."""
     OBJ_DIR.mkdir(exist_ok=True)
     sources = sorted(CSRC.glob("*.hip"))
     if not sources:
         raise RuntimeError(f"no HIP sources under {CSRC}")
     jobs = jobs or min(8, os.cpu_count() or 4)
-    # runtime.hip carries the source digest, so it is rebuilt every time
+    # runtime.hip and the host extension carry the source digest, so they are
+    # rebuilt every time
     digest = (f'-DMI355X_SOURCE_HASH="{_source_hash()}"',)
+    _build_host(digest)
     with ThreadPoolExecutor(max_workers=jobs) as pool:
         objs = list(pool.map(lambda s: _compile(s, force, digest if s.name == "runtime.hip" else ()), sources))
     tmp = LIB_PATH.with_suffix(".so.tmp")

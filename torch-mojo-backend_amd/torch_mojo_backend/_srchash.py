@@ -17,7 +17,7 @@ INCLUDE = PKG_DIR.parent / "include"
 
 
 def source_files() -> list[Path]:
-    files = list(CSRC.glob("*.hip")) + list(CSRC.glob("*.h")) + list(INCLUDE.glob("*.h"))
+    files = list(CSRC.glob("*.hip")) + list(CSRC.glob("*.h")) + list(CSRC.glob("host/*.cpp")) + list(INCLUDE.glob("*.h"))
     return sorted(files, key=lambda f: (f.parent.name, f.name))
 
 

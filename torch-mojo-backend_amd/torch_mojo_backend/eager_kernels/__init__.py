@@ -28,10 +28,27 @@ c_i64 = ctypes.c_int64
 c_double = ctypes.c_double
 c_vp = ctypes.c_void_p
 c_char_p = ctypes.c_char_p
-P_i64 = ctypes.POINTER(ctypes.c_int64)
-P_int = ctypes.POINTER(ctypes.c_int)
-P_vp = ctypes.POINTER(ctypes.c_void_p)
-P_double = ctypes.POINTER(ctypes.c_double)
+
+
+def _array_of(item):
+    """ctypes parameter type of an array argument: a pointer or array of
+    `item`, None, or a tuple or list of numbers (as the native calls take)."""
+    pointer = ctypes.POINTER(item)
+
+    class Array:
+        @classmethod
+        def from_param(cls, value):
+            if isinstance(value, (tuple, list)):
+                value = (item * max(len(value), 1))(*value)
+            return pointer.from_param(value)
+
+    return Array
+
+
+P_i64 = _array_of(c_i64)
+P_int = _array_of(c_int)
+P_vp = _array_of(c_vp)
+P_double = _array_of(c_double)
 
 
 class AdamWTensor(ctypes.Structure):
@@ -291,6 +308,49 @@ def _load() -> ctypes.CDLL:
             " `python torch-mojo-backend_amd/build.py`"
         )
     return lib
+
+
+HOST_PATH = Path(__file__).resolve().parent / "_host.so"
+_HOST = None
+
+
+def host():
+    """The native host module (csrc/host), loaded on first use and checked
+    against the sources beside it like the kernel library."""
+    global _HOST
+    if _HOST is None:
+        import importlib.machinery
+        import importlib.util
+
+        if not HOST_PATH.exists():
+            raise KernelLibraryError(
+                f"{HOST_PATH} is missing: build it with `python torch-mojo-backend_amd/build.py`"
+                " (or __graft_entry__.build())"
+            )
+        loader = importlib.machinery.ExtensionFileLoader("_host", str(HOST_PATH))
+        mod = importlib.util.module_from_spec(importlib.util.spec_from_loader("_host", loader))
+        loader.exec_module(mod)
+        built, expected = mod.source_hash(), _expected_source_hash()
+        if expected is not None and built != expected:
+            raise KernelLibraryError(
+                f"{HOST_PATH} was built from other sources (digest {built}, sources {expected}): rebuild it with"
+                " `python torch-mojo-backend_amd/build.py`"
+            )
+        _HOST = mod
+    return _HOST
+
+
+class _NativeLibrary:
+    """The library's entry points as native calls: the ctypes functions'
+    names, arguments and results without the per-argument conversions."""
+
+    def __init__(self, cdll):
+        native = host()
+        for name in SIGNATURES:
+            fn = getattr(cdll, name)
+            if native.bind(name, ctypes.cast(fn, c_vp).value):
+                fn = getattr(native, name)
+            setattr(self, name, fn)
 
 
 def _expected_source_hash():
@@ -582,11 +642,28 @@ def lib() -> ctypes.CDLL:
     return _LIB
 
 
+_NATIVE = None
+
+
+def native_lib():
+    """`lib()` for the op wrappers: the same entry points, called natively.
+    Deferred launches are issued first here too."""
+    global _NATIVE
+    if _pending:
+        flush_pending()
+    if _NATIVE is None:
+        cdll = lib()
+        if not isinstance(cdll, ctypes.CDLL):
+            return cdll  # a stand-in (host-only tests)
+        _NATIVE = _NativeLibrary(cdll)
+    return _NATIVE
+
+
 def set_library_for_tests(replacement) -> object:
     """Swap the library object (host-only tests); returns the previous one."""
-    global _LIB
+    global _LIB, _NATIVE
     previous = _LIB
-    _LIB = replacement
+    _LIB, _NATIVE = replacement, None
     return previous
 
 

@@ -23,7 +23,8 @@ import os
 
 import torch
 
-from . import AdamWTensor, Deferred, check, defer, flush_pending, lazy, lazy_scale, lib, take_pending
+from . import AdamWTensor, Deferred, check, defer, flush_pending, lazy, lazy_scale, take_pending
+from . import native_lib as lib
 from . import lazy_live as _lazy_pending
 from . import pending_scale as _pending_scale
 from ..mojo_device.torch_mojo_tensor import (
@@ -31,6 +32,7 @@ from ..mojo_device.torch_mojo_tensor import (
     TorchMojoTensor,
     _alloc_bytes,
     compute_contiguous,
+    host as _host,
     row_major_strides,
 )
 
@@ -60,7 +62,11 @@ RED = dict(sum=0, mean=1, max=2, min=3, norm2=4, sumsq=5, amax=6, prod=7, any=8,
 # ---------------------------------------------------------------------------
 # small helpers
 # ---------------------------------------------------------------------------
-def _i64(values) -> ctypes.Array:
+_i64 = tuple  # an array argument of a native call
+
+
+def _i64_array(values) -> ctypes.Array:
+    """An array argument of any length (the multi-tensor calls)."""
     values = tuple(int(v) for v in values)
     return (ctypes.c_int64 * max(len(values), 1))(*values)
 
@@ -84,7 +90,7 @@ def _require(x, what="tensor"):
 
 
 def _alloc(shape, dtype, device: int) -> MT:
-    return MT._alloc(shape, dtype, device)
+    return _host().alloc(shape, dtype, device)
 
 
 def _workspace(nbytes: int, device: int):
@@ -510,6 +516,9 @@ def _view_strides(old_shape, old_strides, new_shape):
 
 def fast_aten_view(self, size):
     t = _require(self)
+    out = _host().reshape_contiguous(t, size)
+    if out is not None:
+        return out
     shape = _infer_size(size, t._numel)
     if t._is_contiguous:
         return MT._view_of(t, shape, row_major_strides(shape), t._offset, True)
@@ -538,8 +547,7 @@ def fast_aten_as_strided(self, size, stride, storage_offset=None):
 
 
 def fast_aten_alias(self):
-    t = _require(self)
-    return MT._view_of(t, t._shape, t._strides, t._offset, t._is_contiguous)
+    return _host().alias(self)
 
 
 fast_aten_detach = fast_aten_alias
@@ -553,15 +561,7 @@ def fast_aten_t(self):
 
 
 def fast_aten_transpose(self, dim0, dim1):
-    t = _require(self)
-    nd = len(t._shape)
-    if nd == 0:
-        return fast_aten_alias(t)
-    d0, d1 = _norm_dim(dim0, nd), _norm_dim(dim1, nd)
-    shape, strides = list(t._shape), list(t._strides)
-    shape[d0], shape[d1] = shape[d1], shape[d0]
-    strides[d0], strides[d1] = strides[d1], strides[d0]
-    return MT._view_of(t, shape, strides, t._offset)
+    return _host().transpose(self, dim0, dim1)
 
 
 def fast_aten_permute(self, dims):
@@ -644,9 +644,9 @@ def fast_aten_split_with_sizes(self, split_sizes, dim=0):
     d = _norm_dim(dim, len(t._shape))
     if sum(split_sizes) != t._shape[d]:
         raise RuntimeError("split_with_sizes expects split_sizes to sum exactly to the dim size")
-    outs, start = [], 0
+    outs, start, narrow = [], 0, _host().narrow
     for s in split_sizes:
-        outs.append(fast_aten_slice(t, d, start, start + s))
+        outs.append(narrow(t, d, start, s))
         start += s
     return outs
 
@@ -705,22 +705,20 @@ def _map_call(opcode, out: MT, inputs, s0=0.0, s1=0.0):
     if out._numel == 0:
         return out
     nin = len(inputs)
-    ptrs = (ctypes.c_void_p * 3)()
-    dts = (ctypes.c_int * 3)()
+    ptrs, dts = [None, None, None], [0, 0, 0]
     strides = list(out._strides)
     for j, (x, dt) in enumerate(inputs):
         if x is None:
-            ptrs[j] = None
             dts[j] = _code(dt)
             strides.extend([0] * len(shape))
         else:
             ptrs[j] = x._ptr
             dts[j] = _code(x._dtype)
-            strides.extend(_broadcast_strides(x, shape))
+            strides.extend(x._strides if x._shape == shape else _broadcast_strides(x, shape))
     check(
         "mi355x_map",
         lib().mi355x_map(
-            opcode, out._ptr, _code(out._dtype), nin, ptrs, dts, _i64(strides), _i64(shape),
+            opcode, out._ptr, _code(out._dtype), nin, ptrs, dts, strides, shape,
             len(shape), float(s0), float(s1), _STREAM,
         ),
     )
@@ -1255,7 +1253,7 @@ def fast_aten_cat(tensors, dim=0):
             "mi355x_foreach_apply",
             lib().mi355x_foreach_apply(
                 0, _ptr_array(ptrs), _ptr_array([x._ptr for x in ts_nonempty]), None, None,
-                _i64([x._numel for x in ts_nonempty]), len(ts_nonempty), _code(dtype), 1.0, None, _STREAM,
+                _i64_array([x._numel for x in ts_nonempty]), len(ts_nonempty), _code(dtype), 1.0, None, _STREAM,
             ),
         )
         return out
@@ -1416,27 +1414,23 @@ def _gemm(out: MT, a: MT, b: MT, bias=None, beta=0, batch=1, round_out=False, ro
     b, brs, bcs, bbs = _gemm_operand(b, rank)
     c_rs = out._strides[-2] if m > 1 else n
     c_bs = out._strides[0] if rank == 3 else 0
-    ws = lib().mi355x_gemm_workspace_bytes(a._ptr, ars, acs, abs_, b._ptr, brs, bcs, bbs,
-                                           _code(a._dtype), batch, m, n, k)
-    hold, wptr = _workspace(ws, a._device)
-    flags = (1 if beta else 0) | (2 if round_out else 0)
-    check(
-        "mi355x_gemm",
-        lib().mi355x_gemm_ex(
-            out._ptr, _code(out._dtype), c_rs, c_bs,
-            a._ptr, ars, acs, abs_,
-            b._ptr, brs, bcs, bbs,
-            _code(a._dtype), bias._ptr if bias is not None else None,
-            _code(bias._dtype) if bias is not None else 0, flags,
-            rowsum._ptr if rowsum is not None else None, _code(rowsum._dtype) if rowsum is not None else 0,
-            batch, m, n, k, ws_ptr_or_none(wptr), ws, _STREAM,
-        ),
-    )
+    _gemm_launch(out, c_rs, c_bs, a, ars, acs, abs_, b, brs, bcs, bbs, bias,
+                 (1 if beta else 0) | (2 if round_out else 0), rowsum, batch, m, n, k)
     return out
 
 
-def ws_ptr_or_none(p):
-    return p if p else None
+def _gemm_launch(out, c_rs, c_bs, a, ars, acs, abs_, b, brs, bcs, bbs, bias, flags, rowsum, batch, m, n, k):
+    """mi355x_gemm_ex on operands with the given strides."""
+    code, kernels = DTYPE_CODE[a._dtype], lib()
+    ws = kernels.mi355x_gemm_workspace_bytes(a._ptr, ars, acs, abs_, b._ptr, brs, bcs, bbs, code, batch, m, n, k)
+    hold, wptr = _workspace(ws, a._device)
+    rc = kernels.mi355x_gemm_ex(
+        out._ptr, _code(out._dtype), c_rs, c_bs, a._ptr, ars, acs, abs_, b._ptr, brs, bcs, bbs, code,
+        bias._ptr if bias is not None else None, _code(bias._dtype) if bias is not None else 0, flags,
+        rowsum._ptr if rowsum is not None else None, _code(rowsum._dtype) if rowsum is not None else 0,
+        batch, m, n, k, wptr, ws, _STREAM,
+    )
+    check("mi355x_gemm", rc)
 
 
 # ---------------------------------------------------------------------------
@@ -1631,8 +1625,13 @@ def linear_forward(x: MT, w: MT, b) -> MT:
     """out[..., N] = x[..., K] @ w[N, K]^T (+ b), one GEMM with the bias
     in its epilogue (aten_fast.py:8755-8812 counterpart)."""
     n, k = w._shape
+    out = _alloc(x._shape[:-1] + (n,), x._dtype, x._device)
+    if (x._is_contiguous and w._is_contiguous and n > 1 and k > 1 and out._numel and x._dtype == w._dtype
+            and (b is None or b._strides[-1] == 1)):
+        # dense operands: their strides are known, no views are needed
+        _gemm_launch(out, n, 0, x, k, 1, 0, w, 1, k, 0, b, 0, None, 1, out._numel // n, n, k)
+        return out
     x2 = _rows_view(x)
-    out = _alloc(tuple(x._shape[:-1]) + (n,), x._dtype, x._device)
     o2 = MT._view_of(out, (x2._shape[0], n), (n, 1), 0, True)
     wt = MT._view_of(w, (k, n), (w._strides[1], w._strides[0]), w._offset)
     if b is not None and b._strides[-1] == 1:
@@ -2109,7 +2108,7 @@ def _add_lazy(a: MT, b: MT, alpha, inplace: bool):
 # scaled dot-product attention (aten_fast.py:7462-7839, 9102-9211)
 # ---------------------------------------------------------------------------
 def _bhs(t: MT):
-    return _i64(t._strides[:3])
+    return t._strides[:3]
 
 
 _FUSED_FA_HEAD_DIMS = (32, 64, 128)  # the MFMA forward + backward
@@ -2645,7 +2644,7 @@ def foreach_apply(opname, a_list, b_list=None, c_list=None, scalars=None, s0=0.0
             opcode, _ptr_array([x._ptr for x in a]),
             _ptr_array([x._ptr for x in b]) if b is not None else None,
             _ptr_array([x._ptr for x in c]) if c is not None else None,
-            sc, _i64([x._numel for x in a]), n, _code(dt), float(s0),
+            sc, _i64_array([x._numel for x in a]), n, _code(dt), float(s0),
             ts._ptr if ts is not None else None, _STREAM,
         ),
     )
@@ -2708,7 +2707,7 @@ def fast_aten__foreach_norm(self, ord=2, dtype=None):
     buf = _alloc((n,), out_dtype, ts[0]._device)
     _mark_cat_ready(buf)
     outs = [MT._view_of(buf, (), (), i, True) for i in range(n)]
-    numels = _i64([t._numel for t in ts])
+    numels = _i64_array([t._numel for t in ts])
     ws = lib().mi355x_foreach_norm_workspace_bytes(numels, n)
     hold, wptr = _workspace(ws, ts[0]._device)
     check(

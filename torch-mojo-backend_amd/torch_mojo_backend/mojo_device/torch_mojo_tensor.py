@@ -24,11 +24,7 @@ dispatcher); ops without a direct entry are redispatched to the
 
 from __future__ import annotations
 
-import math
-
 import torch
-
-_MAX_RANK = 8
 
 # torch dtype -> kernel-library dtype code (include/mi355x_kernels.h)
 DTYPE_CODE = {
@@ -51,12 +47,35 @@ _STORAGE_DEVICES: dict[int, torch.device] = {}
 _TORCH_DEVICES: dict[int, torch.device] = {}
 
 
+class _HostOnUse:
+    """The native host module (csrc/host), set up when it is first used."""
+
+    def __getattr__(self, name):
+        global _host
+        from ..eager_kernels import host
+
+        mod = host()
+        sizes = {d: d.itemsize for d in vars(torch).values() if isinstance(d, torch.dtype)}
+        mod.setup(TorchMojoTensor, torch, storage_device, torch_device_of, _retry_bytes, sizes)
+        mod.reset()
+        _host = mod
+        return getattr(mod, name)
+
+
+_host = _HostOnUse()
+
+
+def host():
+    return _host
+
+
 def set_storage_kind_for_tests(kind: str) -> str:
     """Switch holder allocation between "cuda" and "cpu"; returns the old kind."""
     global _STORAGE_KIND
     previous = _STORAGE_KIND
     _STORAGE_KIND = kind
     _STORAGE_DEVICES.clear()
+    _host.reset()
     return previous
 
 
@@ -108,20 +127,19 @@ def compute_contiguous(shape, strides) -> bool:
 
 
 def _alloc_bytes(nbytes: int, device: int) -> torch.Tensor:
-    """Allocate `nbytes` (at least 1) on the storage device.
+    """`nbytes` (at least 1) on the storage device."""
+    return _host.alloc_bytes(nbytes, device)
 
-    On OOM the caching allocator's free blocks are released and the
-    allocation retried once, the counterpart of the reference's
+
+def _retry_bytes(size: int, device: int) -> torch.Tensor:
+    """The allocation after an OOM: the caching allocator's free blocks are
+    released and it is tried once more, the counterpart of the reference's
     drain-and-retry (torch_mojo_tensor.py:213-244)."""
     dev = storage_device(device)
-    size = max(int(nbytes), 1)
-    try:
-        return torch.empty(size, dtype=torch.uint8, device=dev)
-    except torch.OutOfMemoryError:
-        if dev.type == "cuda":
-            torch.cuda.synchronize(dev)
-            torch.cuda.empty_cache()
-        return torch.empty(size, dtype=torch.uint8, device=dev)
+    if dev.type == "cuda":
+        torch.cuda.synchronize(dev)
+        torch.cuda.empty_cache()
+    return torch.empty(size, dtype=torch.uint8, device=dev)
 
 
 _DISPATCH = None
@@ -152,47 +170,12 @@ class TorchMojoTensor(torch.Tensor):
 
     @classmethod
     def _make(cls, holder, ptr, shape, strides, offset, dtype, device, contiguous=None):
-        shape = tuple(shape)
-        strides = tuple(strides)
-        tdev = torch_device_of(device)
-        res = torch.Tensor._make_wrapper_subclass(
-            cls,
-            shape,
-            strides=strides,
-            storage_offset=offset,
-            dtype=dtype,
-            layout=torch.strided,
-            device=tdev,
-            requires_grad=False,
-        )
-        res._holder = holder
-        res._ptr = ptr
-        res._shape = shape
-        res._strides = strides
-        res._offset = offset
-        res._dtype = dtype
-        res._itemsize = dtype.itemsize
-        res._numel = math.prod(shape)
-        res._device = device
-        res._torch_device = tdev
-        res._is_contiguous = (
-            compute_contiguous(shape, strides) if contiguous is None else contiguous
-        )
-        return res
+        return _host.make(holder, ptr, shape, strides, offset, dtype, device, contiguous)
 
     @classmethod
     def _alloc(cls, shape, dtype, device: int) -> "TorchMojoTensor":
         """A new contiguous uninitialised tensor (one allocation)."""
-        shape = tuple(int(s) for s in shape)
-        if len(shape) > _MAX_RANK:
-            raise NotImplementedError(
-                f"mojo tensors support at most rank {_MAX_RANK}, got {len(shape)}"
-            )
-        numel = math.prod(shape)
-        holder = _alloc_bytes(numel * dtype.itemsize, device)
-        return cls._make(
-            holder, holder.data_ptr(), shape, row_major_strides(shape), 0, dtype, device, True
-        )
+        return _host.alloc(tuple(shape), dtype, device)
 
     @classmethod
     def _alloc_strided(cls, shape, strides, dtype, device: int) -> "TorchMojoTensor":
@@ -208,10 +191,7 @@ class TorchMojoTensor(torch.Tensor):
     @classmethod
     def _view_of(cls, base, shape, strides, offset, contiguous=None) -> "TorchMojoTensor":
         """Zero-copy view sharing `base`'s holder; `offset` is absolute."""
-        ptr = base._ptr + (offset - base._offset) * base._itemsize
-        return cls._make(
-            base._holder, ptr, shape, strides, offset, base._dtype, base._device, contiguous
-        )
+        return _host.view_of(base, shape, strides, offset, contiguous)
 
     @classmethod
     def _from_cpu(cls, cpu_tensor: torch.Tensor, device: int) -> "TorchMojoTensor":
