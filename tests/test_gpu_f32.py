@@ -3,7 +3,7 @@
 import pytest
 import torch
 
-from abi import call, dev, host, lib, p, workspace
+from abi import bhs, call, dev, host, lib, p, workspace
 
 pytestmark = pytest.mark.gpu
 
@@ -39,3 +39,90 @@ def test_gemm_f32_tiles_and_splits(kernels, layout, m, n, k, batch, shift):
              1, batch, m, n, k, p(ws), ws_n, None)
         err = (host(tc).double() - exp).abs()
         assert bool((err <= bound).all()), (ws_n, float((err / bound).max()))
+
+
+def _attention_bounds(q, k, v, do, causal, scale):
+    """(O, LSE, dQ, dK, dV) in 64 bits, and what f32 sums and products may be
+    off by: u = 2^-24; a score D + 4 roundings of sum |q||k|, a probability
+    twice the row's largest such error and 8 u for exp2 and the
+    normalisation, sums of n terms n + 3 roundings of their absolute sum."""
+    u, d, n, m = 2.0 ** -24, q.shape[-1], k.shape[-2], q.shape[-2]
+    s, sa = q @ k.transpose(-2, -1) * scale, q.abs() @ k.abs().transpose(-2, -1) * scale
+    if causal:
+        keep = torch.arange(n)[None, :] <= torch.arange(m)[:, None]
+        s, sa = s.masked_fill(~keep, float("-inf")), sa.masked_fill(~keep, 0.0)
+    es = (d + 4) * u * sa.amax(-1, keepdim=True)
+    pr = torch.softmax(s, -1)
+    rel = 2 * es + 8 * u
+    o, oa = pr @ v, pr @ v.abs()
+    eo = (rel + (n + 8) * u) * oa
+    lse = torch.logsumexp(s, -1)
+    el = es[..., 0] + (n + 8) * u + 8 * u * lse.abs()
+    dp, dpa = do @ v.transpose(-2, -1), do.abs() @ v.abs().transpose(-2, -1)
+    di, dia = (do * o).sum(-1, keepdim=True), (do * o).abs().sum(-1, keepdim=True)
+    ds = pr * (dp - di)
+    edi = (d + 4) * u * dia + (do.abs() * eo).sum(-1, keepdim=True)
+    relp = rel + el[..., None]
+    eds = pr * ((relp + 8 * u) * (dp - di).abs() + (d + 8) * u * dpa + edi + 8 * u * (dp.abs() + di.abs()))
+    t = lambda x: x.transpose(-2, -1)  # noqa: E731
+    out = {"o": (o, eo), "lse": (lse, el),
+           "dq": (scale * (ds @ k), scale * ((eds + (n + 8) * u * ds.abs()) @ k.abs())),
+           "dk": (scale * (t(ds) @ q), scale * (t(eds + (m + 8) * u * ds.abs()) @ q.abs())),
+           "dv": (t(pr) @ do, t((relp + (m + 8) * u) * pr) @ do.abs())}
+    return out
+
+
+@pytest.mark.parametrize("d", [32, 64, 128])
+@pytest.mark.parametrize("causal", [True, False])
+@pytest.mark.parametrize("sq,skv,layout", [(1, 1, "bhsd"), (16, 17, "bshd"), (33, 33, "bshd"), (63, 65, "bhsd"),
+                                           (100, 40, "bshd"), (40, 130, "bshd"), (255, 255, "split"),
+                                           (256, 256, "split"), (70, 70, "odd")])
+def test_attention_f32_matrix_cores(kernels, d, causal, sq, skv, layout):
+    """f32 attention at the edges of its 16-row waves, 32-row tiles and 64-row
+    blocks, more keys than queries and fewer, rows inside a fused projection,
+    and ("odd") rows that are not 16-byte aligned, which the general kernels
+    take."""
+    B, H, scale = 2, 3, 0.3 / d ** 0.5 * 3
+    gen = torch.Generator().manual_seed(d * 1000 + sq * 7 + skv)
+    q, do = (torch.randn(B, H, sq, d, generator=gen) for _ in range(2))
+    k, v = (torch.randn(B, H, skv, d, generator=gen) for _ in range(2))
+
+    def store(x, pad):
+        if layout == "bhsd":
+            return dev(x)
+        t = torch.zeros(x.shape[0], x.shape[2], x.shape[1] * d + pad, device="cuda")
+        w = t[..., : x.shape[1] * d].unflatten(-1, (x.shape[1], d)).transpose(1, 2)
+        w.copy_(x)
+        return w
+
+    pad = {"split": 2 * H * d, "odd": 1}.get(layout, 0)
+    tq, tk, tv, tdo = (store(x, pad) for x in (q, k, v, do))
+    o, dq = (store(torch.zeros_like(q), pad) for _ in range(2))
+    dk, dv = (store(torch.zeros_like(k), pad) for _ in range(2))
+    lse = torch.empty(B, H, sq, device="cuda")
+    call("mi355x_attn_fwd_gen", p(o), bhs(o), p(lse), p(tq), bhs(tq), p(tk), bhs(tk), p(tv), bhs(tv), B, H, H, sq, skv,
+         d, scale, int(causal), 0, 0, None)
+    ws_n = lib().mi355x_attn_bwd_gen_workspace_bytes(B, H, H, sq, skv, d)
+    ws = workspace(ws_n)
+    call("mi355x_attn_bwd_gen", p(dq), bhs(dq), p(dk), bhs(dk), p(dv), bhs(dv), p(tdo), bhs(tdo), p(tq), bhs(tq),
+         p(tk), bhs(tk), p(tv), bhs(tv), p(o), bhs(o), p(lse), B, H, H, sq, skv, d, scale, int(causal), 0, 0, p(ws),
+         ws_n, None)
+    want = _attention_bounds(*(x.double() for x in (q, k, v, do)), causal, scale)
+    for name, got in (("o", o), ("lse", lse), ("dq", dq), ("dk", dk), ("dv", dv)):
+        ref, bound = want[name]
+        err = (host(got).double() - ref).abs()
+        assert bool((err <= bound).all()), (name, float((err / bound.clamp_min(1e-300)).max()))
+
+
+def test_attention_f32_infinities_and_nan(kernels, mojo):
+    """A NaN or infinite element shows where it shows on the CPU: in its own
+    query's row, and in every later query's through its key."""
+    gen = torch.Generator().manual_seed(5)
+    for bad in (float("nan"), float("inf")):
+        q, k, v = (torch.randn(1, 2, 70, 64, generator=gen) for _ in range(3))
+        q[0, 0, 7, 3] = bad
+        v[0, 1, 40, 5] = bad
+        got = torch.nn.functional.scaled_dot_product_attention(q.to("mojo"), k.to("mojo"), v.to("mojo"), is_causal=True)
+        got = got.cpu()
+        assert got[0, 0, 7].isnan().all() and got[0, 0, 8:].isfinite().all() and got[0, 0, :7].isfinite().all()
+        assert not got[0, 1, 40:, 5].isfinite().any() and got[0, 1, :32].isfinite().all()

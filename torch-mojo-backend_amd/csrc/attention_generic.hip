@@ -1,6 +1,8 @@
-// Fused attention for the inputs the MFMA kernels do not take: f32 inputs,
-// any head_dim up to 256, and the backward of grouped-K/V-head and
-// sliding-window attention.  Everything is computed in f32.
+// Fused attention for the inputs the MFMA kernels do not take: any head_dim
+// up to 256, f32 with grouped K/V heads or a window, and the backward of
+// grouped-K/V-head and sliding-window attention.  Everything is computed in
+// f32.  Plain f32 attention at head_dim 32, 64 and 128 goes on from these
+// entry points to the matrix cores (attention_f32.hip).
 //
 // Semantics are those of attention.hip: S = scale Q K^T over the visible keys
 // (top-left causal: key j visible to query i iff j <= i; with a window w > 0
@@ -20,6 +22,7 @@
 // row group of a wave reads the same address, a broadcast).
 #include <math.h>
 
+#include "attention_f32.h"
 #include "common.h"
 
 namespace mi {
@@ -372,6 +375,19 @@ GenArgs gen_args(const void* q, const int64_t* q_bhs, const void* k, const int64
   return a;
 }
 
+// The operands for attention_f32.hip, where the call is one it can take: f32,
+// a K/V head for each query head, no window.
+bool f32_args(const GenArgs& a, int dtype, AttnF32* f) {
+  if (dtype != MI355X_F32 || a.H != a.HK || a.window != 0) return false;
+  *f = AttnF32{(float*)a.o, a.o_b, a.o_h, a.o_s, a.lse,
+               (const float*)a.q, a.q_b, a.q_h, a.q_s, (const float*)a.k, a.k_b, a.k_h, a.k_s,
+               (const float*)a.v, a.v_b, a.v_h, a.v_s, (const float*)a.dout, a.do_b, a.do_h, a.do_s,
+               (float*)a.dq, a.dq_b, a.dq_h, a.dq_s, (float*)a.dk, a.dk_b, a.dk_h, a.dk_s,
+               (float*)a.dv, a.dv_b, a.dv_h, a.dv_s, a.delta, a.B, a.H, a.Sq, a.Skv,
+               a.scale_log2, a.scale, a.causal};
+  return true;
+}
+
 }  // namespace
 }  // namespace mi
 
@@ -388,6 +404,11 @@ extern "C" int mi355x_attn_fwd_gen(void* o, const int64_t* o_bhs, float* lse, co
   GenArgs a = gen_args(q, q_bhs, k, k_bhs, v, v_bhs, batch, heads, kv_heads, sq, skv, d, scale, causal, window);
   a.o = o; a.o_b = o_bhs[0]; a.o_h = o_bhs[1]; a.o_s = o_bhs[2];
   a.lse = lse;
+  AttnF32 f;
+  if (f32_args(a, dtype, &f)) {
+    rc = attn_f32_fwd(f, d, (hipStream_t)stream);
+    if (rc >= 0) return rc;
+  }
   MI_GEN_DISPATCH(dtype, d, gen_fwd_launch, a, (hipStream_t)stream);
 }
 
@@ -439,5 +460,10 @@ extern "C" int mi355x_attn_bwd_gen(void* dq, const int64_t* dq_bhs, void* dk, co
   a.dk = dk; a.dk_b = dk_bhs[0]; a.dk_h = dk_bhs[1]; a.dk_s = dk_bhs[2];
   a.dv = dv; a.dv_b = dv_bhs[0]; a.dv_h = dv_bhs[1]; a.dv_s = dv_bhs[2];
   a.delta = (float*)workspace;
+  AttnF32 f;
+  if (f32_args(a, dtype, &f)) {
+    rc = attn_f32_bwd(f, d, (hipStream_t)stream);
+    if (rc >= 0) return rc;
+  }
   MI_GEN_DISPATCH(dtype, d, gen_bwd_launch, a, (hipStream_t)stream);
 }
