@@ -12,8 +12,11 @@
 //   k-contiguous operand: tile [row][32 k], 16-byte chunks XOR-swizzled by
 //     (row >> 1) & 7; one 16-byte read is a fragment's operand for 4 MFMAs;
 //   m/n-contiguous operand: tile [k][rows]; one read of F consecutive rows at
-//     one k is one operand of F fragments, so fragment i holds rows F*r + i
-//     and the result's rows (columns) are permuted the same way.
+//     one k is one operand of F fragments, so fragment i holds rows F*r + i.
+// k-contiguous tiles hold their rows in that order too, so a lane's results
+// are F adjacent columns of C and leave in one store (16384 x 3072 x 768 with
+// both operands k-contiguous: 705 -> 655 us, 118 TFLOP/s; n-contiguous B
+// 127 TFLOP/s).
 // VEC loads tiles 16 bytes per lane, which needs 16-byte aligned rows and a
 // contiguous extent that is a multiple of 4; other operands are loaded 4
 // bytes per lane into the same tiles (still an eighth of the MFMA time).
@@ -31,11 +34,20 @@ constexpr int kBK = 32;   // k per stage
 constexpr int kNT = 256;  // 4 waves, 2 x 2
 
 __device__ __forceinline__ int swz(int row) { return (row >> 1) & 7; }
+constexpr int kCPR = kBK / 4;  // 16-byte chunks per k-contiguous row
+
+// Row of the operand at row p of a k-contiguous tile: within each wave's
+// F fragments, row F * r + i lies at 16 i + r, so that fragment i holds rows
+// F * r + i as with an m/n-contiguous operand and a lane's results are
+// adjacent columns of C.
+template <int F>
+__device__ __forceinline__ int src_row(int p) { return p / (16 * F) * (16 * F) + (p & 15) * F + (p / 16) % F; }
 
 // Loads a ROWS x 32-k tile of an operand that is contiguous in k.
 template <int ROWS, bool VEC>
 struct LoadK {
-  static constexpr int RPI = VEC ? 8 : 2;             // rows per wave instruction
+  static constexpr int RPI = VEC ? 64 / kCPR : 64 / kBK;  // rows per wave instruction
+  static constexpr int F = ROWS / 32;
   static constexpr int ITERS = ROWS / (RPI * 4);      // instructions per wave
   const float* src[VEC ? ITERS : 1];
   const float* base;
@@ -47,10 +59,10 @@ struct LoadK {
     if constexpr (VEC) {
       // swz repeats every 16 rows and a wave's instructions are 32 rows
       // apart, so a lane's chunk is the same for all of them
-      const int r = wave * RPI + lane / 8;
-      kof = ((lane % 8) ^ swz(r)) * 4;
+      const int r = wave * RPI + lane / kCPR;
+      kof = ((lane % kCPR) ^ swz(r)) * 4;
 #pragma unroll
-      for (int it = 0; it < ITERS; ++it) src[it] = b + min(r0 + r + it * RPI * 4, n - 1) * ld_;
+      for (int it = 0; it < ITERS; ++it) src[it] = b + min(r0 + src_row<F>(r + it * RPI * 4), n - 1) * ld_;
     } else {
       base = b, ld = ld_, row0 = r0, rows = n;
     }
@@ -65,9 +77,9 @@ struct LoadK {
       const int lane = threadIdx.x & 63;
 #pragma unroll 4
       for (int it = 0; it < ITERS; ++it) {
-        const int r = (it * 4 + wave_id()) * 2 + lane / 32, p = lane % 32;
+        const int r = (it * 4 + wave_id()) * RPI + lane / kBK, p = lane % kBK;
         const int64_t k = k0 + (((p >> 2) ^ swz(r)) << 2) + (p & 3);
-        dma_b32(base + min(row0 + r, rows - 1) * ld + (k < kend ? k : k0), lds + it * 1024);
+        dma_b32(base + min(row0 + src_row<F>(r), rows - 1) * ld + (k < kend ? k : k0), lds + it * 1024);
       }
     }
   }
@@ -195,31 +207,40 @@ __global__ void __launch_bounds__(kNT, 2) gemm_f32_tile(GemmArgs g, int tiles_m,
   for (int64_t k0 = kbeg; k0 < kend; k0 += kBK, cur ^= 1) {
     __builtin_amdgcn_s_waitcnt(0x0f70);  // vmcnt(0): this stage has landed
     __syncthreads();
+    const char* at = lds + cur * STAGE;
+    const char* bt = at + HALF;
+    // All of the stage's operands are read before its MFMAs, and the next
+    // stage's loads are issued in the shadow of the first reads: one LDS
+    // latency a stage.
+    float a[kBK / 16][F][4], b[kBK / 16][F][4];
+    frags<TILE, A_K, F>(at, wm * W, 0, a[0]);
+    frags<TILE, B_K, F>(bt, wn * W, 0, b[0]);
     if (k0 + kBK < kend) {  // into the stage that every wave has finished reading
       la.issue(k0 + kBK, kend, lds + (cur ^ 1) * STAGE);
       lb.issue(k0 + kBK, kend, lds + (cur ^ 1) * STAGE + HALF);
     }
-    const char* at = lds + cur * STAGE;
-    const char* bt = at + HALF;
-    const bool tail = k0 + kBK > kend;
 #pragma unroll
-    for (int ks = 0; ks < kBK / 16; ++ks) {
-      float a[F][4], b[F][4];
-      frags<TILE, A_K, F>(at, wm * W, ks, a);
-      frags<TILE, B_K, F>(bt, wn * W, ks, b);
-      if (tail) {  // both operands: what lies past the end may be inf or NaN
+    for (int ks = 1; ks < kBK / 16; ++ks) {
+      frags<TILE, A_K, F>(at, wm * W, ks, a[ks]);
+      frags<TILE, B_K, F>(bt, wn * W, ks, b[ks]);
+    }
+    if (k0 + kBK > kend) {  // both operands: what lies past the end may be inf or NaN
+#pragma unroll
+      for (int ks = 0; ks < kBK / 16; ++ks) {
         const int64_t k = k0 + ks * 16 + 4 * lg;
-        mask(a, k, kend);
-        mask(b, k, kend);
+        mask(a[ks], k, kend);
+        mask(b[ks], k, kend);
       }
+    }
+#pragma unroll
+    for (int ks = 0; ks < kBK / 16; ++ks)
 #pragma unroll
       for (int s = 0; s < 4; ++s)
 #pragma unroll
         for (int i = 0; i < F; ++i)
 #pragma unroll
           for (int j = 0; j < F; ++j)
-            acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x4f32(a[i][s], b[j][s], acc[i][j], 0, 0, 0);
-    }
+            acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x4f32(a[ks][i][s], b[ks][j][s], acc[i][j], 0, 0, 0);
   }
 
   // lane (lg, lr) holds rows 4 lg + e of fragment row i and column lr of
@@ -229,7 +250,7 @@ __global__ void __launch_bounds__(kNT, 2) gemm_f32_tile(GemmArgs g, int tiles_m,
   int64_t cols[F];
 #pragma unroll
   for (int j = 0; j < F; ++j) {
-    cols[j] = col0 + (B_K ? j * 16 + lr : F * lr + j);
+    cols[j] = col0 + F * lr + j;
     bias[j] = (!g.part && g.bias && cols[j] < g.n) ? ld_any(g.bias, g.bias_dt, cols[j]) : 0.f;
   }
   float* P = nullptr;
@@ -240,12 +261,12 @@ __global__ void __launch_bounds__(kNT, 2) gemm_f32_tile(GemmArgs g, int tiles_m,
   const bool beta = g.beta && !g.part;
   typedef float vec __attribute__((ext_vector_type(F)));
   // F adjacent columns per lane leave in one store where they are aligned
-  const bool wide = !B_K && P && !beta && cols[F - 1] < g.n && (rs % F) == 0 && ((uintptr_t)P % (4 * F)) == 0;
+  const bool wide = P && !beta && cols[F - 1] < g.n && (rs % F) == 0 && ((uintptr_t)P % (4 * F)) == 0;
 #pragma unroll
   for (int i = 0; i < F; ++i)
 #pragma unroll
     for (int e = 0; e < 4; ++e) {
-      const int64_t row = row0 + (A_K ? i * 16 + 4 * lg + e : F * (4 * lg + e) + i);
+      const int64_t row = row0 + F * (4 * lg + e) + i;
       if (row >= g.m) continue;
       if (wide) {
         vec v;
@@ -272,24 +293,25 @@ struct PlanF32 {
 };
 
 // The tile size and the number of K splits with the least estimated time: the
-// rounds of 256 CUs times a block's MFMA time (two resident blocks of a CU
-// share its matrix units, so each counts as a round), plus about 1.5 us of
-// load latency per block that nothing hides in a short K loop, plus, with
-// splits, the partials' traffic and the summing launch.
+// rounds of 256 CUs (blocks that share a CU share its matrix units) times a
+// block's time at the rate that one block per CU was measured at (4096 x 3072,
+// K = 768: 128 tiles in 3 rounds 181 us, 64 tiles in 12 rounds 208 us), plus,
+// with splits, the summing launch (the partials of 4096 x 768 in 3 splits:
+// 8 us).
 PlanF32 plan_f32(int64_t batch, int64_t m, int64_t n, int64_t k) {
   PlanF32 best{128, 1, k};
   double tbest = 1e30;
   for (int tile = 128; tile >= 64; tile -= 64) {
     const int64_t tiles = ((m + tile - 1) / tile) * ((n + tile - 1) / tile) * batch;
-    const double per_k = 2.0 * tile * tile / (tile == 128 ? 560e3 : 500e3);  // us per k at a CU's rate
+    const double per_k = 2.0 * tile * tile / (tile == 128 ? 440e3 : 375e3);  // us
     for (int64_t sp = 1; sp <= 32 && (sp == 1 || (k / sp >= 128 && tiles < 4 * kCUs)); ++sp) {
       int64_t chunk = (k + sp - 1) / sp;
       chunk = (chunk + kBK - 1) / kBK * kBK;
       const int64_t s = (k + chunk - 1) / chunk;
       if (s != sp) continue;  // the same split as a smaller sp
       const double rounds = (double)((tiles * s + kCUs - 1) / kCUs);
-      double t = rounds * per_k * (double)(s > 1 ? chunk : k) + 1.5;
-      if (s > 1) t += 4.0 + (double)(2 * s + 1) * 4.0 * (double)(batch * m * n) / 5e6;
+      double t = rounds * per_k * (double)(s > 1 ? chunk : k);
+      if (s > 1) t += 3.0 + (double)(s + 1) * 4.0 * (double)(batch * m * n) / 6e6;
       if (t < tbest * 0.98) tbest = t, best = PlanF32{tile, (int)s, s > 1 ? chunk : k};
     }
   }
@@ -298,8 +320,25 @@ PlanF32 plan_f32(int64_t batch, int64_t m, int64_t n, int64_t k) {
 
 template <int TILE, bool A_K, bool B_K, bool VEC>
 int launch(const GemmArgs& g, int tiles_m, dim3 grid, hipStream_t s) {
-  constexpr size_t lds = 2 * 2 * (size_t)TILE * kBK * 4;  // 64 KB at most: no opt-in needed
-  gemm_f32_tile<TILE, A_K, B_K, VEC><<<grid, kNT, lds, s>>>(g, tiles_m, tiles_m <= g.tiles_n ? 1 : 0);
+  constexpr size_t lds = 2 * 2 * (size_t)TILE * kBK * 4;  // 64 KB at most
+  size_t bytes = lds;
+  if (TILE == 128 && VEC) {
+    // Two blocks fit a CU.  When the last pair of rounds has only one block
+    // per CU to give, the CUs whose two blocks end together take two again
+    // while others idle; with the LDS of one block per CU the rounds are whole
+    // (4096 x 3072, K = 768, 768 blocks: 221 -> 181 us; with more rounds two
+    // per CU are faster, 1024 x 50257: 760 against 831 us, and with 4-byte
+    // loads, whose latency a second block hides, K = 50257: 995 against 1093).
+    const int64_t blocks = (int64_t)grid.x * grid.y;
+    if (blocks <= 4 * kCUs && (blocks + kCUs - 1) / kCUs < 2 * ((blocks + 2 * kCUs - 1) / (2 * kCUs))) {
+      constexpr int alone = 88 * 1024;  // more than half of a CU's 160 KB
+      static const bool ok = hipFuncSetAttribute((const void*)gemm_f32_tile<TILE, A_K, B_K, VEC>,
+                                                 hipFuncAttributeMaxDynamicSharedMemorySize, alone) == hipSuccess;
+      if (!ok) return fail(MI355X_ELAUNCH, "mi355x_gemm: cannot reserve %d bytes of LDS", alone);
+      bytes = alone;
+    }
+  }
+  gemm_f32_tile<TILE, A_K, B_K, VEC><<<grid, kNT, bytes, s>>>(g, tiles_m, tiles_m <= g.tiles_n ? 1 : 0);
   return check_launch("mi355x_gemm");
 }
 
