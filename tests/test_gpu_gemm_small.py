@@ -35,3 +35,33 @@ def test_gemm_64_tiles(kernels, dtype, layout, m, n, k, batch):
     a, b, u = A.double(), B.double(), (k + 3) * 2.0 ** -23
     assert bool(((host(c).double() - a @ b).abs() <= u * (a.abs() @ b.abs())).all())
     assert bool(((host(rows).double() - a.sum(2)).abs() <= u * a.abs().sum(2)).all())
+
+
+@pytest.mark.parametrize("m,n,layout", [(65, 67, "NT"), (1030, 2051, "NN"), (4100, 2301, "NT"), (8200, 5003, "NN")])
+@pytest.mark.parametrize("c_dtype,flags", [(torch.bfloat16, 0), (torch.float16, 0), (torch.float32, 0), (torch.float32, 2),
+                                           (torch.bfloat16, 1)])
+def test_gemm_stores_at_any_alignment(kernels, m, n, layout, c_dtype, flags):
+    """Partial tiles of each block configuration into rows of C at every
+    alignment (odd row stride, a base shifted by one element): every element
+    of C right, nothing else written.  k = 64 sums of exact products, rounded
+    once to the output type (and through bf16 with ROUND)."""
+    k, ld, shift = 64, n + 3 + n % 2, 1
+    gen = torch.Generator().manual_seed(m + n)
+    A, B, bias = (torch.randn(*s, generator=gen).bfloat16() for s in ((m, k), (k, n), (n,)))
+    ta, tb, tbias = dev(A), dev((B.t() if layout[1] == "T" else B).contiguous()), dev(bias)
+    b_rs, b_cs = (n, 1) if layout[1] == "N" else (1, k)
+    store = torch.full((shift + m * ld,), 3.0, dtype=c_dtype, device="cuda")
+    args = (p(ta), k, 1, 0, p(tb), b_rs, b_cs, 0, 1)
+    ws_n = lib().mi355x_gemm_workspace_bytes(*args, 1, m, n, k)
+    ws = workspace(ws_n) if ws_n else None
+    call("mi355x_gemm_ex", p(store) + shift * store.element_size(), CODE[c_dtype], ld, 0, *args, p(tbias), 1, flags, None,
+         0, 1, m, n, k, p(ws), ws_n, None)
+    got = store[shift:].view(m, ld)
+    assert bool((got[:, n:] == 3.0).all()) and float(store[0]) == 3.0
+    exact = ta.double() @ dev(B).double() + tbias.double() + (3.0 if flags == 1 else 0.0)
+    ulp = {torch.bfloat16: 2.0 ** -8, torch.float16: 2.0 ** -11, torch.float32: 2.0 ** -24}[c_dtype]
+    if flags == 2:
+        ulp = 2.0 ** -8
+        assert torch.equal(got[:, :n], got[:, :n].bfloat16().float())
+    bound = ulp * exact.abs() + (k + 3) * 2.0 ** -23 * (ta.double().abs() @ dev(B).double().abs() + 4)
+    assert bool(((got[:, :n].double() - exact).abs() <= bound).all())

@@ -264,30 +264,23 @@ __device__ __forceinline__ void wait_stage(int64_t later) {
   else if constexpr (LATER > 0) wait_stage<LATER - 1, PER_STAGE>(later);
 }
 
-// Write one wave's accumulators to C (pointing at the wave tile's first
-// element), adding the preloaded bias and, with BETA, the old C.  Offsets
-// inside the tile are 32-bit (the host checks the row stride); EDGE adds the
-// bounds checks that only partial tiles need.  Each store instruction covers
-// four 16-column runs, and the j loop fills whole 128-byte lines.
-template <typename CT, typename T, bool BETA, bool EDGE, bool ROUND, int TM, int TN>
-__device__ __forceinline__ void store_tile(CT* __restrict__ C, int c_rs, const f32x4 (&acc)[TM][TN],
-                                           const float (&bias)[TN], int rows_left, int cols_left, int lr,
-                                           int lg) {
+// C += a wave's accumulators plus the preloaded bias, element by element (C
+// points at the wave tile's first element).  Offsets inside the tile are
+// 32-bit (the host checks the row stride).
+template <typename CT, int TM, int TN>
+__device__ __forceinline__ void add_tile(CT* __restrict__ C, int c_rs, const f32x4 (&acc)[TM][TN],
+                                         const float (&bias)[TN], int rows_left, int cols_left, int lr, int lg) {
 #pragma unroll
   for (int i = 0; i < TM; ++i)
 #pragma unroll
     for (int e = 0; e < 4; ++e) {
       const int r = i * 16 + lg * 4 + e;
-      if (EDGE && r >= rows_left) continue;
+      if (r >= rows_left) continue;
       CT* row = C + r * c_rs;
 #pragma unroll
       for (int j = 0; j < TN; ++j) {
         const int c = j * 16 + lr;
-        if (EDGE && c >= cols_left) continue;
-        float v = acc[i][j][e] + bias[j];
-        if (BETA) v += (float)row[c];
-        if (ROUND) v = (float)(T)v;
-        row[c] = (CT)v;
+        if (c < cols_left) row[c] = (CT)(acc[i][j][e] + bias[j] + (float)row[c]);
       }
     }
 }
@@ -342,22 +335,54 @@ __device__ __forceinline__ void store_tile_lds(CT* __restrict__ C, int c_rs, con
   }
 }
 
-template <typename CT, typename T, int TM, int TN>
-__device__ __forceinline__ void store_any(CT* C, int c_rs, const f32x4 (&acc)[TM][TN], const float (&bias)[TN],
-                                          bool beta, bool round, int rows_left, int cols_left, int lr, int lg) {
-  const bool edge = rows_left < TM * 16 || cols_left < TN * 16;
-#define ST(B, E, R) store_tile<CT, T, B, E, R>(C, c_rs, acc, bias, rows_left, cols_left, lr, lg)
-  if (round) {  // round-through stores are only used without beta
-    if (edge) ST(false, true, true);
-    else ST(false, false, true);
-  } else if (beta) {
-    if (edge) ST(true, true, false);
-    else ST(true, false, false);
-  } else {
-    if (edge) ST(false, true, false);
-    else ST(false, false, false);
+// The same through the slab for partial tiles and for rows of C that are not
+// 16-byte aligned, whose 16-byte stores the hardware splits: still far fewer
+// instructions than storing element by element (logits of 50257 columns,
+// 16384 x 768: 1463 -> 1402 us; splitting each row at its 16-byte boundary
+// instead took 1544; 1000 x 3072 at K = 768, which ended with the last row of
+// tiles: 16.7 -> 13.1).  Columns past the last whole 16 bytes leave one by
+// one.  Cached stores, so that the lines that two waves share are merged.
+template <typename CT, typename T, bool ROUND, int TM, int TN>
+__device__ __forceinline__ void store_tile_edge(CT* __restrict__ C, int c_rs, const f32x4 (&acc)[TM][TN],
+                                                const float (&bias)[TN], float* slab, int rows_left, int cols_left,
+                                                int lr, int lg, int lane) {
+  constexpr int WN = TN * 16, LD = WN + kSlabPad;
+  constexpr int E = 16 / sizeof(CT);
+  const int cols = min(cols_left, WN);
+#pragma unroll
+  for (int i = 0; i < TM; ++i) {
+    if (i * 16 >= rows_left) break;
+#pragma unroll
+    for (int j = 0; j < TN; ++j)
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        float v = acc[i][j][e] + bias[j];
+        if (ROUND) v = (float)(T)v;
+        slab[(lg * 4 + e) * LD + j * 16 + lr] = v;
+      }
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+#pragma unroll
+    for (int it = 0; it < 16 * (WN / E) / 64; ++it) {
+      const int ch = it * 64 + lane, r = ch / (WN / E), c = (ch % (WN / E)) * E;
+      if (i * 16 + r >= rows_left || c + E > cols) continue;
+      const float* src = slab + r * LD + c;
+      struct Out { CT v[E]; } out;  // aligned as its elements are
+#pragma unroll
+      for (int e = 0; e < E; ++e) out.v[e] = (CT)src[e];
+      *(Out*)(C + (i * 16 + r) * c_rs + c) = out;
+    }
+    if (cols % E != 0)
+#pragma unroll
+      for (int it = 0; it < 16 * E / 64; ++it) {
+        const int q = it * 64 + lane, r = q / E, c = cols / E * E + q % E;
+        if (i * 16 + r < rows_left && c < cols) C[(i * 16 + r) * c_rs + c] = (CT)slab[r * LD + c];
+      }
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
   }
-#undef ST
 }
 
 // RS: also sum A's rows over k, from the fragments the MFMAs consume, with
@@ -587,7 +612,7 @@ __global__ void __launch_bounds__(64 * TileCfg<CFG>::WGM * TileCfg<CFG>::WGN, Ti
     if (rows_left == WM && cols_left == WN && (g.n & 3) == 0 && ((uintptr_t)g.part & 15) == 0)
       store_tile_lds<float, T, false, false>(P, (int)g.n, acc, bias, slab, lr, lg, lane);
     else
-      store_any<float, T>(P, (int)g.n, acc, bias, false, false, rows_left, cols_left, lr, lg);
+      store_tile_edge<float, T, false>(P, (int)g.n, acc, bias, slab, rows_left, cols_left, lr, lg, lane);
     return;
   }
 #pragma unroll
@@ -608,9 +633,18 @@ __global__ void __launch_bounds__(64 * TileCfg<CFG>::WGM * TileCfg<CFG>::WGN, Ti
     else store_tile_lds<float, T, false, true>((float*)Cb, c_rs, acc, bias, slab, lr, lg, lane);
     return;
   }
-  if (g.c_dt == MI355X_BF16) store_any<bf16, T>((bf16*)Cb, c_rs, acc, bias, g.beta, false, rows_left, cols_left, lr, lg);
-  else if (g.c_dt == MI355X_F32) store_any<float, T>((float*)Cb, c_rs, acc, bias, g.beta, rnd, rows_left, cols_left, lr, lg);
-  else store_any<f16, T>((f16*)Cb, c_rs, acc, bias, g.beta, false, rows_left, cols_left, lr, lg);
+  if (g.beta) {
+    if (g.c_dt == MI355X_BF16) add_tile<bf16>((bf16*)Cb, c_rs, acc, bias, rows_left, cols_left, lr, lg);
+    else if (g.c_dt == MI355X_F32) add_tile<float>((float*)Cb, c_rs, acc, bias, rows_left, cols_left, lr, lg);
+    else add_tile<f16>((f16*)Cb, c_rs, acc, bias, rows_left, cols_left, lr, lg);
+    return;
+  }
+#define EDGE(CT, R) store_tile_edge<CT, T, R>((CT*)Cb, c_rs, acc, bias, slab, rows_left, cols_left, lr, lg, lane)
+  if (g.c_dt == MI355X_BF16) EDGE(bf16, false);
+  else if (g.c_dt == MI355X_F16) EDGE(f16, false);
+  else if (rnd) EDGE(float, true);
+  else EDGE(float, false);
+#undef EDGE
 }
 
 // Launch one kernel instantiation; the first launch of each opts it into
