@@ -247,24 +247,48 @@ int64_t rs_slots_of(int cfg, int64_t n) {
   return (n + c.bn - 1) / c.bn * c.wgn;
 }
 
-// Pick the configuration that finishes in the least time: whole rounds of
-// the CUs' block slots (two C128 blocks or one C256 block per CU) times the
-// per-round time measured on gfx950 at K = 768..3072 (a C256 round does
-// twice a C128 round's work in 1.82x its time).  An m-contiguous A (a weight
-// gradient dY^T X) reads both operands through transposing LDS reads, which
-// C256 tiles halve per flop: when both sides span a 256 tile it takes them,
-// in 32-k stages (the 50304 x 768 embedding gradient: 1.53 -> 1.35 ms, the
-// 768 x 3072 one 105 -> 84 us with 7 K splits).  Then split K when the
+// Time of `blocks` blocks of a configuration, in units of a full round of C128
+// (two blocks on each CU, 0.0141 us per k).  A round that gives a CU one block
+// of the two that fit it is shorter (us at K = 768 unless given, C128 / C192 /
+// C256 tiles: 4096 x 2304 24.2 / 20.2 / 22.8, 8192 x 2304 40.2 / 32.7 / 46.5,
+// 8192 x 3072 45.9 / 40.5 / 48.3, 16384 x 2304 70.7 / 59.7 / 72.2, 16384 x
+// 3072 96.4 / 83.7 / 82.0, 2048 x 2304 14.8 / 14.1 / 20.7, 4096 x 768 11.3 /
+// 13.9 / 20.7, 16384 x 1024 at K = 1024 38.0 / 49.3 / 33.8).
+double rounds_of(int cfg, int64_t blocks) {
+  if (cfg == 1) return 1.8 * (double)((blocks + kCUs - 1) / kCUs);
+  const double two = cfg == 2 ? 1.45 : 1.0, one = cfg == 2 ? 0.95 : 0.72;
+  const int64_t last = blocks % (2 * kCUs);
+  return two * (double)(blocks / (2 * kCUs)) + (last == 0 ? 0.0 : last <= kCUs ? one : two);
+}
+
+// Pick the configuration that finishes in the least time.  An m-contiguous A
+// (a weight gradient dY^T X) reads both operands through transposing LDS
+// reads, which C256 tiles halve per flop: when both sides span a 256 tile it
+// takes them, in 32-k stages (the 50304 x 768 embedding gradient: 1.53 -> 1.35
+// ms, the 768 x 3072 one 105 -> 84 us with 7 K splits).  Then split K when the
 // output alone cannot fill the chip.
 Plan plan_gemm(int64_t batch, int64_t m, int64_t n, int64_t k, bool a_kcontig, bool b_kcontig) {
   Plan best{0, 1, k};
   const int64_t t128 = tiles_of(0, batch, m, n), t256 = tiles_of(1, batch, m, n), t192 = tiles_of(2, batch, m, n);
-  const double c128 = (double)((t128 + 2 * kCUs - 1) / (2 * kCUs));
-  const double c256 = 1.82 * (double)((t256 + kCUs - 1) / kCUs);
-  const double c192 = 1.5 * (double)((t192 + 2 * kCUs - 1) / (2 * kCUs));
-  double cbest = c128;
-  if (t256 >= kCUs && c256 < cbest) best.cfg = 1, cbest = c256;
-  if (b_kcontig && t192 >= kCUs && c192 < cbest) best.cfg = 2, cbest = c192;
+  double cbest = rounds_of(0, t128);
+  // at least three quarters of the CUs busy (2048 x 6912, 216 C256 tiles, K = 1152: 40.4 -> 32.9 us)
+  const int64_t fill = kCUs * 3 / 4;
+  if (t256 >= (a_kcontig ? fill : kCUs) && rounds_of(1, t256) < cbest) best.cfg = 1, cbest = rounds_of(1, t256);
+  if (b_kcontig && t192 >= fill && rounds_of(2, t192) < cbest) best.cfg = 2, cbest = rounds_of(2, t192);
+  if (a_kcontig && t128 > kCUs && 2 * t128 < 3 * kCUs && k >= 4096) {
+    // A long K under a round that is little more than half full: K splits, if
+    // they pay for their partial sums (4096 x 1152 at K = 6912: 97 us; 75 in 3
+    // splits of C256, 79 in 2 of C192, 84 in 3 of C128).
+    double tbest = 0.9 * cbest * 0.0141 * (double)k;
+    for (int cfg = 0; cfg <= (b_kcontig ? 2 : 1); ++cfg)
+      for (int64_t sp = 2; sp <= 4; ++sp) {
+        const int64_t chunk = ((k + sp - 1) / sp + 63) / 64 * 64;
+        const double t = rounds_of(cfg, tiles_of(cfg, batch, m, n) * sp) * 0.0141 * (double)chunk + 3.0 +
+                         (double)(sp + 1) * 4.0 * (double)(batch * m * n) / 6e6;
+        if (t < tbest) tbest = t, best = Plan{cfg, (int)((k + chunk - 1) / chunk), chunk};
+      }
+    if (best.splits > 1) return best;
+  }
   // Weight gradients (m-contiguous A) take the 32-k C256 stages when their
   // 256x256 tiles fill the CUs (wte: 50304 x 768); smaller ones take
   // split-K C128, whose K ranges the XCD-ordered grid keeps in one or two
