@@ -65,3 +65,25 @@ def test_gemm_stores_at_any_alignment(kernels, m, n, layout, c_dtype, flags):
         assert torch.equal(got[:, :n], got[:, :n].bfloat16().float())
     bound = ulp * exact.abs() + (k + 3) * 2.0 ** -23 * (ta.double().abs() @ dev(B).double().abs() + 4)
     assert bool(((got[:, :n].double() - exact).abs() <= bound).all())
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("layout", ["NT", "NN", "TN", "TT"])
+@pytest.mark.parametrize("m,n,k,batch", [(700, 6000, 768, 1), (2500, 10007, 520, 2), (130, 33000, 136, 1)])
+def test_gemm_groups_of_tile_rows(kernels, dtype, layout, m, n, k, batch):
+    """B beyond 8 MB: the tiles are walked in groups of rows, the last group a
+    partial one.  Each element of C against products exact in f64."""
+    gen = torch.Generator().manual_seed(m + n + k)
+    A, B = (torch.randn(batch, *s, generator=gen).to(dtype) for s in ((m, k), (k, n)))
+    ta = dev((A.transpose(1, 2) if layout[0] == "T" else A).contiguous())
+    tb = dev((B.transpose(1, 2) if layout[1] == "T" else B).contiguous())
+    a_rs, a_cs = (k, 1) if layout[0] == "N" else (1, m)
+    b_rs, b_cs = (n, 1) if layout[1] == "N" else (1, k)
+    args = (p(ta), a_rs, a_cs, m * k, p(tb), b_rs, b_cs, k * n)
+    ws_n = lib().mi355x_gemm_workspace_bytes(*args, CODE[dtype], batch, m, n, k)
+    ws = workspace(ws_n) if ws_n else None
+    c = torch.full((batch, m, n), float("nan"), device="cuda")
+    call("mi355x_gemm_ex", p(c), 0, n, m * n, *args, CODE[dtype], None, 0, 0, None, 0, batch, m, n, k, p(ws), ws_n, None)
+    for i in range(batch):
+        a, b = dev(A[i]).double(), dev(B[i]).double()
+        assert bool(((c[i].double() - a @ b).abs() <= (k + 3) * 2.0 ** -23 * (a.abs() @ b.abs())).all())

@@ -20,6 +20,7 @@ struct GemmArgs {
   float* part;     // split-K partials [splits][batch][m][n] (f32) or null
   int64_t kchunk;  // K per split
   int tiles_n;     // tiles along n
+  int group;       // tile rows walked together (1: row by row)
   int batch;       // batch count (grid.y = splits * batch)
   int ab_dt;       // operand dtype (for rounding through it)
   int round_c;     // round C (and the row sums) through ab_dt before storing

@@ -508,7 +508,7 @@ extern "C" int mi355x_gemm_ex(void* c, int c_dtype, int64_t c_rs, int64_t c_bs, 
   MI_REQUIRE(c && a && b, "mi355x_gemm: null pointer");
   hipStream_t s = (hipStream_t)stream;
   GemmArgs g{c, c_dtype, c_rs, c_bs, a, a_rs, a_cs, a_bs, b, b_rs, b_cs, b_bs, bias, bias_dtype,
-             beta, m, n, k, nullptr, k, 1, 1, ab_dtype, round_c, a_rowsum, a_rowsum_dtype, nullptr};
+             beta, m, n, k, nullptr, k, 1, 1, 1, ab_dtype, round_c, a_rowsum, a_rowsum_dtype, nullptr};
   if (ab_dtype == MI355X_F32) {
     MI_REQUIRE(!a_rowsum && !round_c, "mi355x_gemm: row sums and ROUND need 16-bit operands");
     return gemm_f32_launch(g, batch, workspace, ws_bytes, s);
