@@ -87,3 +87,52 @@ def test_gemm_groups_of_tile_rows(kernels, dtype, layout, m, n, k, batch):
     for i in range(batch):
         a, b = dev(A[i]).double(), dev(B[i]).double()
         assert bool(((c[i].double() - a @ b).abs() <= (k + 3) * 2.0 ** -23 * (a.abs() @ b.abs())).all())
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("layout", ["NT", "NN", "TN", "TT"])
+@pytest.mark.parametrize("m,n,k,rows", [(520, 300, 8200, False), (2100, 776, 8192, False), (3600, 3850, 2048, False),
+                                        (1540, 3090, 4104, True), (1540, 3090, 4160, False)])
+def test_gemm_long_k(kernels, dtype, layout, m, n, k, rows):
+    """256x256 tiles of four waves: whole K and splits, one to three stages
+    past the ring's length, a ragged last stage, edges of the tile, and the
+    row sums that take eight waves instead."""
+    gen = torch.Generator().manual_seed(m + 3 * n + k)
+    n8, m8 = (n + 7) // 8 * 8, (m + 7) // 8 * 8  # rows in place: strides of whole 16 bytes
+    A, B = (torch.randn(*s, generator=gen).to(dtype) for s in ((m8, k), (k, n8)))
+    ta = dev((A.t() if layout[0] == "T" else A).contiguous())
+    tb = dev((B.t() if layout[1] == "T" else B).contiguous())
+    a_rs, a_cs = (k, 1) if layout[0] == "N" else (1, m8)
+    b_rs, b_cs = (n8, 1) if layout[1] == "N" else (1, k)
+    args = (p(ta), a_rs, a_cs, 0, p(tb), b_rs, b_cs, 0)
+    ws_n = lib().mi355x_gemm_workspace_bytes(*args, CODE[dtype], 1, m, n, k)
+    ws = workspace(ws_n) if ws_n else None
+    c = torch.full((m, n), float("nan"), device="cuda")
+    sums = torch.full((m,), float("nan"), device="cuda") if rows else None
+    call("mi355x_gemm_ex", p(c), 0, n, 0, *args, CODE[dtype], None, 0, 0, p(sums) if rows else None, 0, 1, m, n, k, p(ws),
+         ws_n, None)
+    a, b, u = dev(A[:m]).double(), dev(B[:, :n]).double(), (k + 3) * 2.0 ** -23
+    assert bool(((c.double() - a @ b).abs() <= u * (a.abs() @ b.abs())).all())
+    if rows:
+        assert bool(((sums.double() - a.sum(1)).abs() <= u * a.abs().sum(1)).all())
+
+
+@pytest.mark.parametrize("layout", ["NT", "NN", "TN", "TT"])
+@pytest.mark.parametrize("k", [2048, 2056, 2112, 2176, 2240])
+def test_gemm_long_k_ends(kernels, layout, k):
+    """Every place in the ring for the last stage, whole and ragged, against
+    the same product in f64 (K from 2048: the four-wave tiles)."""
+    m, n = 3608, 3848
+    gen = torch.Generator().manual_seed(k)
+    A, B = (torch.randn(*s, generator=gen).bfloat16() for s in ((m, k), (k, n)))
+    ta = dev((A.t() if layout[0] == "T" else A).contiguous())
+    tb = dev((B.t() if layout[1] == "T" else B).contiguous())
+    a_rs, a_cs = (k, 1) if layout[0] == "N" else (1, m)
+    b_rs, b_cs = (n, 1) if layout[1] == "N" else (1, k)
+    args = (p(ta), a_rs, a_cs, 0, p(tb), b_rs, b_cs, 0)
+    ws_n = lib().mi355x_gemm_workspace_bytes(*args, 1, 1, m, n, k)
+    ws = workspace(ws_n) if ws_n else None
+    c = torch.full((m, n), float("nan"), device="cuda")
+    call("mi355x_gemm_ex", p(c), 0, n, 0, *args, 1, None, 0, 0, None, 0, 1, m, n, k, p(ws), ws_n, None)
+    a, b = dev(A).double(), dev(B).double()
+    assert bool(((c.double() - a @ b).abs() <= (k + 3) * 2.0 ** -23 * (a.abs() @ b.abs())).all())

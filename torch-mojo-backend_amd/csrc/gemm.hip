@@ -218,7 +218,7 @@ __global__ void __launch_bounds__(256) pack_k_contig_v8(uint16_t* __restrict__ d
 // planning
 // ---------------------------------------------------------------------------
 struct Plan {
-  int cfg;  // 0 = C128, 1 = C256, 2 = C192, 3 = C256 in 32-k stages
+  int cfg;  // 0 = C128, 1 = C256, 2 = C192, 3 = C256W, 4 = C64
   int splits;
   int64_t kchunk;
 };
@@ -261,12 +261,16 @@ double rounds_of(int cfg, int64_t blocks) {
   return two * (double)(blocks / (2 * kCUs)) + (last == 0 ? 0.0 : last <= kCUs ? one : two);
 }
 
-// Pick the configuration that finishes in the least time.  An m-contiguous A
-// (a weight gradient dY^T X) reads both operands through transposing LDS
-// reads, which C256 tiles halve per flop: when both sides span a 256 tile it
-// takes them, in 32-k stages (the 50304 x 768 embedding gradient: 1.53 -> 1.35
-// ms, the 768 x 3072 one 105 -> 84 us with 7 K splits).  Then split K when the
-// output alone cannot fill the chip.
+// Time of a plan, in us: its rounds, with K splits the partial sums' way out
+// and back and the launch that adds them.
+double plan_time(double rounds, int64_t chunk, int64_t splits, int64_t outputs) {
+  return rounds * 0.0141 * (double)chunk + (splits > 1 ? 3.0 + (double)(splits + 1) * 4.0 * (double)outputs / 6e6 : 0.0);
+}
+
+int64_t chunk_of(int64_t k, int64_t splits) { return ((k + splits - 1) / splits + 63) / 64 * 64; }
+
+// Pick the configuration that finishes in the least time, then split K when
+// the output alone cannot fill the chip.
 Plan plan_gemm(int64_t batch, int64_t m, int64_t n, int64_t k, bool a_kcontig, bool b_kcontig) {
   Plan best{0, 1, k};
   const int64_t t128 = tiles_of(0, batch, m, n), t256 = tiles_of(1, batch, m, n), t192 = tiles_of(2, batch, m, n);
@@ -282,19 +286,40 @@ Plan plan_gemm(int64_t batch, int64_t m, int64_t n, int64_t k, bool a_kcontig, b
     double tbest = 0.9 * cbest * 0.0141 * (double)k;
     for (int cfg = 0; cfg <= (b_kcontig ? 2 : 1); ++cfg)
       for (int64_t sp = 2; sp <= 4; ++sp) {
-        const int64_t chunk = ((k + sp - 1) / sp + 63) / 64 * 64;
-        const double t = rounds_of(cfg, tiles_of(cfg, batch, m, n) * sp) * 0.0141 * (double)chunk + 3.0 +
-                         (double)(sp + 1) * 4.0 * (double)(batch * m * n) / 6e6;
+        const int64_t chunk = chunk_of(k, sp);
+        const double t = plan_time(rounds_of(cfg, tiles_of(cfg, batch, m, n) * sp), chunk, sp, batch * m * n);
         if (t < tbest) tbest = t, best = Plan{cfg, (int)((k + chunk - 1) / chunk), chunk};
       }
-    if (best.splits > 1) return best;
   }
-  // Weight gradients (m-contiguous A) take the 32-k C256 stages when their
-  // 256x256 tiles fill the CUs (wte: 50304 x 768); smaller ones take
-  // split-K C128, whose K ranges the XCD-ordered grid keeps in one or two
-  // L2s (config 2 shapes, TF/s: 768 x 768 646 against 501, 2304 x 768 912
-  // against 839, 768 x 3072 933 against 915).
-  if (!a_kcontig && m >= 256 && n >= 256 && t256 >= kCUs) best.cfg = 3;
+  // C256W from K = 2048: there its faster loop outweighs a slower start and
+  // end (C256 / C256W, us: 8192 x 8192 at K = 1024 139 / 148, 1536 202 / 203,
+  // 3072 376 / 364; 4096 x 12288 at K = 4096 368 / 357).
+  if (best.cfg == 1 && best.splits == 1 && k >= 2048) best.cfg = 3;
+  // An m-contiguous A (a weight gradient dY^T X) reads both operands through
+  // transposing LDS reads, which 256x256 tiles halve per flop: it takes them
+  // when they fill the CUs, or in K splits that do when C128 would leave part
+  // of a single round empty (1536 x 3072 at K = 16384: 288 C128 tiles 233 us, 72
+  // in three splits 160).  Splits have to save 15% by the model, which leaves
+  // out the burst of the partial sums (8192 x 3072 at K = 8192: 400 us in one,
+  // 433 in two).  Smaller outputs take split-K C128, with half the splits
+  // (768 x 768 at K = 16384 33 / 40; 768 x 3072 is 96 / 89 by itself, but a
+  // training step of such layers was 0.3 ms slower for the partial sums).
+  bool planned = false;
+  if (!a_kcontig && m >= 256 && n >= 256 && t128 >= kCUs) {
+    const double r0 = t256 >= kCUs ? 1e30 : rounds_of(0, t128), r1 = rounds_of(1, t256);
+    const double whole = plan_time(r0 < r1 ? r0 : r1, k, 1, 0);
+    double tbest = whole;
+    best = Plan{r0 < r1 ? 0 : k >= 2048 ? 3 : 1, 1, k};
+    for (int64_t sp = 2; sp <= 4 && k / sp >= 512; ++sp) {
+      const int64_t chunk = chunk_of(k, sp);
+      const double t = plan_time(rounds_of(1, t256 * sp), chunk, sp, batch * m * n);
+      if (t < tbest && t < 0.85 * whole) {
+        tbest = t;
+        best = Plan{chunk >= 2048 ? 3 : 1, (int)((k + chunk - 1) / chunk), chunk};
+      }
+    }
+    planned = true;
+  }
   // Outputs of at most two 64x64 tiles per CU with up to 5e9 multiply-adds:
   // their larger tiles leave CUs idle and a k-step takes its latencies, not
   // its MFMA time (us, larger tiles against C64; K = 768 unless given: 77 x
@@ -305,34 +330,16 @@ Plan plan_gemm(int64_t batch, int64_t m, int64_t n, int64_t k, bool a_kcontig, b
   // K = 2048 24.5 / 26.4), or a K long enough to split over all CUs (768 x
   // 768 at K = 8192 24.2 / 24.2, at 16384 33.4 / 40.9; 1024 x 768 at K = 8192
   // 26.4 / 29.6).
-  if (tiles_of(4, batch, m, n) <= 2 * kCUs && (double)(batch * m * n) * (double)k <= 5e9) best.cfg = 4;
-  static const char* forced = getenv("MI355X_GEMM_TILE");  // tuning override: "128", "192", "256" or "256.32"
+  if (tiles_of(4, batch, m, n) <= 2 * kCUs && (double)(batch * m * n) * (double)k <= 5e9) best = Plan{4, 1, k}, planned = false;
+  static const char* forced = getenv("MI355X_GEMM_TILE");  // tuning override: "64", "128", "192", "256" or "257" (C256W)
   if (forced) {
     const double f = atof(forced);
-    best.cfg = f == 256 ? 1 : (f > 256 && !a_kcontig ? 3 : (f == 192 && b_kcontig ? 2 : (f == 64 ? 4 : 0)));
+    best.cfg = f == 256 ? 1 : (f > 256 ? 3 : (f == 192 && b_kcontig ? 2 : (f == 64 ? 4 : 0)));
+    best = Plan{best.cfg, 1, k};
+    planned = false;
   }
   const int64_t tiles = tiles_of(best.cfg, batch, m, n);
-  if (best.cfg == 3 && tiles >= kCUs && k >= 8192) {
-    // One block per CU: a last round that is mostly empty costs a whole
-    // round.  K splits that fill the rounds better win when the gain is
-    // large (the 50304 x 768 embedding gradient, K = 16384: 591 tiles are
-    // 2.3 rounds; two splits make 4.6 of half length: 1.49 -> 1.29 ms plus
-    // a 75 us partial sum, train step -0.12 ms).
-    const double r1 = (double)((tiles + kCUs - 1) / kCUs);
-    int64_t bs = 1;
-    double bcost = r1;
-    for (int64_t sp = 2; sp <= 4; ++sp) {
-      const double c = (double)((tiles * sp + kCUs - 1) / kCUs) / (double)sp + 0.05 * (double)sp;
-      if (c < bcost * 0.9) bs = sp, bcost = c;
-    }
-    if (bs > 1) {
-      int64_t chunk = (k + bs - 1) / bs;
-      chunk = (chunk + 63) / 64 * 64;
-      best.splits = (int)((k + chunk - 1) / chunk);
-      best.kchunk = chunk;
-    }
-  }
-  if (tiles < kCUs && k >= 2048) {
+  if (!planned && best.splits == 1 && tiles < kCUs && k >= 2048) {
     // as many K splits as keep every block in the first round of block
     // slots: a second, partly filled round would double the time
     const int64_t slots = best.cfg == 1 || best.cfg == 3 ? kCUs : 2 * kCUs;  // block slots of the chosen config
@@ -345,6 +352,22 @@ Plan plan_gemm(int64_t batch, int64_t m, int64_t n, int64_t k, bool a_kcontig, b
       chunk = (chunk + 63) / 64 * 64;
       best.splits = (int)((k + chunk - 1) / chunk);
       best.kchunk = chunk;
+    }
+  }
+  // Over a very long K a round of C256W takes 1.4 units against the others'
+  // model (50257 into 768 columns, us, before / C256W: 16384 rows C192 1386 /
+  // 1268, in four splits 1211; 8192 rows C192 977 / in two splits 660; 2048 rows
+  // C128 in 5 splits 204 / in ten 180; but 1000 rows C128 in 10 splits 95 / in
+  // sixteen 112).
+  if (a_kcontig && k >= 8192 && m >= 256 && n >= 256 && best.cfg != 4 && !forced) {
+    const double r = best.cfg == 3 ? 1.4 * (double)((tiles * best.splits + kCUs - 1) / kCUs)
+                                   : rounds_of(best.cfg, tiles * best.splits);
+    double tbest = plan_time(r, best.kchunk, best.splits, batch * m * n);
+    const double whole = plan_time(1.4 * (double)((t256 + kCUs - 1) / kCUs), k, 1, 0);
+    for (int64_t sp = 1; sp <= 10; ++sp) {
+      const int64_t chunk = chunk_of(k, sp);
+      const double t = plan_time(1.4 * (double)((t256 * sp + kCUs - 1) / kCUs), chunk, sp, batch * m * n);
+      if (t < tbest && (sp == 1 || t < 0.85 * whole)) tbest = t, best = Plan{3, (int)((k + chunk - 1) / chunk), chunk};
     }
   }
   return best;
@@ -391,7 +414,8 @@ namespace {
 template <typename T>
 int launch_mfma(GemmArgs g, int64_t batch, const Plan& p, hipStream_t s) {
   const bool kt = g.k % 64 != 0;
-  int rc = kt ? gemm_tiles<T, true>(g, batch, p.cfg, p.splits, s) : gemm_tiles<T, false>(g, batch, p.cfg, p.splits, s);
+  const int cfg = g.rowsum && p.cfg == 3 ? 1 : p.cfg;  // the same tiles; C256W takes no row sums
+  int rc = kt ? gemm_tiles<T, true>(g, batch, cfg, p.splits, s) : gemm_tiles<T, false>(g, batch, cfg, p.splits, s);
   if (rc || !g.part) return rc;
   const int rs_slots = g.rowsum ? (int)(p.splits * rs_slots_of(p.cfg, g.n)) : 0;
   rc = splitk_finish(g, batch, p.splits, rs_slots, s);

@@ -24,6 +24,8 @@
 //         k-contiguous only); N = 768, 2304, 3072 split into whole rounds;
 //   C256: 256x256, 8 waves of 128x64, 128 KB LDS, one block per CU (fewer
 //         LDS bytes per flop; preferred when its tiles fill the CUs evenly);
+//   C256W: 256x256, 4 waves of 128x128, 160 KB LDS, one block per CU, from
+//         K = 2048 where C256 would be taken;
 //   C64: 64x64, 4 waves of 32x32, for outputs too small to fill the CUs
 //         otherwise (one GPT-2 layer of a 77-token prompt: 11.8 -> 6.4 us a
 //         product).
@@ -237,13 +239,13 @@ template <>
 struct TileCfg<2> {  // C192: 128x192, waves of 64x96, 40 KB per stage (k-contiguous B only)
   static constexpr int BM = 128, BN = 192, BK = 64, WGM = 2, WGN = 2, STAGES = 2, MIN_BLOCKS = 2;
 };
-// C256 in 32-k stages, three deep (96 KB): for weight gradients, whose
-// operands are both m/n-contiguous.  Their transposing fragment reads make
-// a 64-k step long; halving it and keeping two stages in flight hides the
-// loads better (gfx950, cfg 2 shapes: 7-13% over 64-k stages).
+// C256W: the same tile by four waves of 128x128, one on each SIMD, for long K.
+// What bounds C256's loop is LDS: its waves of 128x64 read 192 KB a stage (1536
+// cycles) and the loads write 64 KB (512), as long as the MFMAs (2048); these
+// read 128 KB.  Five slots of 32 KB (160 KB).
 template <>
 struct TileCfg<3> {
-  static constexpr int BM = 256, BN = 256, BK = 32, WGM = 2, WGN = 4, STAGES = 3, MIN_BLOCKS = 1;
+  static constexpr int BM = 256, BN = 256, BK = 64, WGM = 2, WGN = 2, STAGES = 2, MIN_BLOCKS = 1;
 };
 
 // C64: 64x64, 4 waves of 32x32, four 16 KB stages, two blocks per CU: for
@@ -387,6 +389,129 @@ __device__ __forceinline__ void store_tile_edge(CT* __restrict__ C, int c_rs, co
   }
 }
 
+// One fragment: rows r0 .. r0 + 15, k substep ks of a stage's tile of ROWS rows.
+template <typename T, int ROWS, bool K_CONTIG>
+__device__ __forceinline__ typename Mfma<T>::frag read_frag(const char* tile, int r0, int ks) {
+  typedef typename Mfma<T>::frag frag;
+  const int lane = threadIdx.x & 63, lr = lane & 15, lg = lane >> 4;
+  if constexpr (K_CONTIG) {
+    return *(const frag*)(tile + (r0 + lr) * 128 + ((ks * 4 + lg) ^ rswz<64>(lr)) * 16);
+  } else {
+    frag f[1];
+    mn_frags<T, ROWS, 1>(tile, r0, ks, f);
+    return f[0];
+  }
+}
+
+// c += a b on accumulators that stay where they are: given the builtin, the
+// compiler moves 256 of them about between the MFMAs of a loop.  The hazard
+// that this hides from it, reading c too soon after, is settle_acc's.
+typedef int i32x4 __attribute__((ext_vector_type(4)));
+__device__ __forceinline__ void mma_acc(f32x4& c, const Mfma<bf16>::frag& a, const Mfma<bf16>::frag& b) {
+  asm volatile("v_mfma_f32_16x16x32_bf16 %0, %1, %2, %0"
+               : "+a"(c) : "v"(__builtin_bit_cast(i32x4, a)), "v"(__builtin_bit_cast(i32x4, b)));
+}
+__device__ __forceinline__ void mma_acc(f32x4& c, const Mfma<f16>::frag& a, const Mfma<f16>::frag& b) {
+  asm volatile("v_mfma_f32_16x16x32_f16 %0, %1, %2, %0"
+               : "+a"(c) : "v"(__builtin_bit_cast(i32x4, a)), "v"(__builtin_bit_cast(i32x4, b)));
+}
+
+// C256W's k loop.  A wave has its SIMD to itself, so nothing hides what it
+// waits for but its own MFMAs: each 32-k substep's fragments are read during
+// the substep before, and the loads of a stage are issued over both substeps
+// of the stage two before it, A's into the slot that the ring has free, B's
+// into the one that A leaves at the barrier between them.  In one burst after
+// that barrier, with four slots, they stalled the wave (8192^3 1112 us; 868).
+// Two or one loads a row took as long in the forward and 7% longer with
+// transposed operands.
+// Against C256 (us): 8192^3 917 -> 869, dX 1074 -> 927, dW 1110 -> 994; 50257
+// columns dX 16384 rows 1468 -> 1268 (C192 1386), dW 1275 -> 1160; 16384 x
+// 4096 at K = 4096 471 -> 461; but at K = 768 83 -> 86 and 74 -> 79: four waves
+// fill and drain a tile more slowly than eight.
+template <typename T, typename C, bool KT, bool A_K, bool B_K, typename LA, typename LB, int TM, int TN>
+__device__ __forceinline__ void wide_loop(const LA& la, const LB& lb, f32x4 (&acc)[TM][TN], char* lds, int64_t kbeg,
+                                          int64_t kend, int wm, int wn) {
+  typedef typename Mfma<T>::frag frag;
+  constexpr int A_BYTES = C::BM * C::BK * 2, STAGE = A_BYTES + C::BN * C::BK * 2, BK = C::BK;
+  constexpr int NA = LA::ITERS, NQ = NA + LB::ITERS, R = TM + TN;
+  constexpr int LPR = 4;  // loads per row of MFMAs: A's in the first substep's first rows, B's in the second's
+  struct Frags { frag a[TM], b[TN]; } f0, f1;
+  auto read = [&](Frags& f, const char* ta, const char* tb, int ks, int lo, int hi) {  // B's first: every row of MFMAs takes them all
+#pragma unroll
+    for (int q = 0; q < R; ++q) {
+      if (q < lo || q >= hi) continue;
+      if (q < TN) f.b[q] = read_frag<T, C::BN, B_K>(tb, wn * TN * 16 + q * 16, ks);
+      else f.a[q - TN] = read_frag<T, C::BM, A_K>(ta, wm * TM * 16 + (q - TN) * 16, ks);
+    }
+  };
+  auto mask = [&](frag& f, int64_t kfrag) {
+    mask_k(f, kfrag, kend);
+    asm volatile("s_nop 3" : "+v"(f));  // an MFMA may read it 2 states later
+  };
+  auto mask_all = [&](Frags& f, int64_t kfrag) {
+#pragma unroll
+    for (int j = 0; j < TN; ++j) mask(f.b[j], kfrag);
+#pragma unroll
+    for (int i = 0; i < TM; ++i) mask(f.a[i], kfrag);
+  };
+  if (kbeg >= kend) return;
+  // stage 0 is in flight
+  if (kbeg + BK < kend) {
+    la.template issue<KT>(kbeg + BK, lds + STAGE, kend);
+    lb.template issue<KT>(kbeg + BK, lds + STAGE + A_BYTES, kend);
+    __builtin_amdgcn_s_waitcnt(vmcnt_imm(NQ));
+  } else {
+    __builtin_amdgcn_s_waitcnt(vmcnt_imm(0));
+  }
+  __syncthreads();
+  read(f0, lds, lds + A_BYTES, 0, 0, R);
+  const int lg = (threadIdx.x & 63) >> 4;
+  // slots of 32 KB in a ring of five: A of stage s in slot 2 s % 5, B in the next
+  char *sa = lds, *sb = lds + A_BYTES;
+  auto next = [&](char* s, int n) {  // n slots on
+    s += n * A_BYTES;
+    return s >= lds + 5 * A_BYTES ? s - 5 * A_BYTES : s;
+  };
+  auto step = [&](int64_t k0, auto tail_c, auto more_c) {
+    constexpr bool tail = decltype(tail_c)::value, more = decltype(more_c)::value;
+    char *const na = next(sa, 2), *const nb = next(sb, 2), *const fre = next(sa, 4);
+    if (tail) mask_all(f0, k0 + lg * 8);
+#pragma unroll
+    for (int i = 0; i < TM; ++i) {
+      if (more) la.template issue_range<KT>(k0 + 2 * BK, fre, kend, i * LPR, (i + 1) * LPR);
+      read(f1, sa, sb, 1, i * R / (TM - 2), (i + 1) * R / (TM - 2));
+      if (i == TM - 1) {
+        // all of this stage is in registers and the next one has landed
+        __builtin_amdgcn_s_waitcnt(vmcnt_imm(more ? NA : 0));
+        __syncthreads();
+      }
+#pragma unroll
+      for (int j = 0; j < TN; ++j) mma_acc(acc[i][j], f0.a[i], f0.b[j]);
+      __builtin_amdgcn_sched_barrier(0);
+    }
+    if (tail) mask_all(f1, k0 + 32 + lg * 8);
+#pragma unroll
+    for (int i = 0; i < TM; ++i) {
+      if (more) lb.template issue_range<KT>(k0 + 2 * BK, sa, kend, i * LPR, (i + 1) * LPR);
+      read(f0, na, nb, 0, i * R / (TM - 1), (i + 1) * R / (TM - 1));  // past the last stage: not used
+#pragma unroll
+      for (int j = 0; j < TN; ++j) mma_acc(acc[i][j], f1.a[i], f1.b[j]);
+      __builtin_amdgcn_sched_barrier(0);
+    }
+    sa = na;
+    sb = nb;
+  };
+  int64_t k0 = kbeg;
+  for (; k0 + 2 * BK < kend; k0 += BK) step(k0, std::false_type{}, std::true_type{});
+  for (; KT ? k0 + BK <= kend : k0 < kend; k0 += BK) step(k0, std::false_type{}, std::false_type{});
+  if (KT && k0 < kend) step(k0, std::true_type{}, std::false_type{});
+  // an MFMA's results may be read 10 states after it
+#pragma unroll
+  for (int i = 0; i < TM; ++i)
+#pragma unroll
+    for (int j = 0; j < TN; ++j) asm volatile("s_nop 15" : "+a"(acc[i][j]));
+}
+
 // RS: also sum A's rows over k, from the fragments the MFMAs consume, with
 // one extra MFMA against a fragment of ones (every column of its 16x16
 // result is the row sum).  With split K the 32-k substeps are dealt round
@@ -501,8 +626,8 @@ __global__ void __launch_bounds__(64 * TileCfg<CFG>::WGM * TileCfg<CFG>::WGN, Ti
     // rows of the first 32-k substep instead, so the load issue no longer
     // stalls the wave in one burst: the forward fc and lm_head launches run
     // 3.4-5.8% faster in the training step (kernel trace, two boxes); the
-    // same spread lost 2-6% on the 128x128 and 128x192 tiles and the 32-k
-    // 256x256 weight-gradient tiles, which keep the single burst.
+    // same spread lost 2-6% on the 128x128 and 128x192 tiles, which keep the
+    // single burst.
     const bool more = k0 + (S - 1) * BK < kend;
     char* const nxt = lds + (cur == 0 ? S - 1 : cur - 1) * STAGE;
     const char* at = lds + cur * STAGE;
@@ -595,9 +720,13 @@ __global__ void __launch_bounds__(64 * TileCfg<CFG>::WGM * TileCfg<CFG>::WGN, Ti
     }
     cur = cur == S - 1 ? 0 : cur + 1;
   };
-  int64_t k0 = kbeg;
-  for (; KT ? k0 + BK <= kend : k0 < kend; k0 += BK) step(k0, std::false_type{});
-  if (KT && k0 < kend) step(k0, std::true_type{});
+  if constexpr (CFG == 3) {
+    wide_loop<T, C, KT, A_K, B_K>(la, lb, acc, lds, kbeg, kend, wm, wn);
+  } else {
+    int64_t k0 = kbeg;
+    for (; KT ? k0 + BK <= kend : k0 < kend; k0 += BK) step(k0, std::false_type{});
+    if (KT && k0 < kend) step(k0, std::true_type{});
+  }
 
   // every wave is past its last LDS read: the stages become store slabs
   __syncthreads();
@@ -671,7 +800,7 @@ template <typename T, int CFG, bool A_K, bool B_K, bool KT, bool RS>
 int launch_kernel(const GemmArgs& g, dim3 grid, hipStream_t s) {
   typedef TileCfg<CFG> C;
   constexpr int NT = 64 * C::WGM * C::WGN;
-  constexpr size_t lds = C::STAGES * (size_t)(C::BM + C::BN) * C::BK * 2;
+  constexpr size_t lds = CFG == 3 ? 163840 : C::STAGES * (size_t)(C::BM + C::BN) * C::BK * 2;
   static bool attr = false;
   if (lds > 65536 && !attr) {
     if (hipFuncSetAttribute((const void*)gemm_tile<T, CFG, A_K, B_K, KT, RS>,
@@ -686,11 +815,7 @@ int launch_kernel(const GemmArgs& g, dim3 grid, hipStream_t s) {
 template <typename T, int CFG, bool KT, bool RS>
 int launch_layout(const GemmArgs& g, dim3 grid, hipStream_t s) {
   const bool ak = g.a_cs == 1, bk = g.b_rs == 1;
-  if constexpr (CFG == 3) {  // chosen for m-contiguous A only
-    if (ak) return fail(MI355X_EINVAL, "mi355x_gemm: 32-k C256 tiles take an m-contiguous A");
-    if (bk) return launch_kernel<T, CFG, false, true, KT, RS>(g, grid, s);
-    return launch_kernel<T, CFG, false, false, KT, RS>(g, grid, s);
-  } else if constexpr (CFG == 2) {  // 192-wide B tiles are only loaded k-contiguous
+  if constexpr (CFG == 2) {  // 192-wide B tiles are only loaded k-contiguous
     if (!bk) return fail(MI355X_EINVAL, "mi355x_gemm: 128x192 tiles need a k-contiguous B");
     if (ak) return launch_kernel<T, CFG, true, true, KT, RS>(g, grid, s);
     return launch_kernel<T, CFG, false, true, KT, RS>(g, grid, s);
@@ -719,7 +844,9 @@ int launch_tile(GemmArgs g, int64_t batch, int splits, hipStream_t s) {
     g.group = (int)(rows < 1 ? 1 : rows > tm ? tm : rows);
   }
   dim3 grid((unsigned)(tm * tn), (unsigned)(batch * splits));
-  if (g.rowsum) return launch_layout<T, CFG, KT, true>(g, grid, s);
+  if constexpr (CFG != 3) {  // which has no row sums
+    if (g.rowsum) return launch_layout<T, CFG, KT, true>(g, grid, s);
+  }
   return launch_layout<T, CFG, KT, false>(g, grid, s);
 }
 
