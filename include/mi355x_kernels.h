@@ -501,10 +501,11 @@ int mi355x_foreach_apply(int op, void* const* a, const void* const* b,
  * B element at b + b*b_bs + k*b_rs + n*b_cs (b_rs == 1 or b_cs == 1),
  * C element at c + b*c_bs + m*c_rs + n (rows contiguous).
  * ab_dtype: F32, BF16 or F16 (A and B share it); c_dtype and bias_dtype:
- * F32/BF16/F16.  Accumulates in f32; bf16/f16 use MFMA.  beta == 1 adds the
+ * F32/BF16/F16.  Accumulates in f32, on MFMA.  beta == 1 adds the
  * existing C (accumulate), beta == 0 overwrites. */
 /* Workspace for the call with these operands (split-K partials, and packed
- * copies of operands that cannot be read in place). */
+ * copies of operands that cannot be read in place; f32 operands: the partials
+ * only, and without a workspace the call runs in one split). */
 int64_t mi355x_gemm_workspace_bytes(const void* a, int64_t a_rs, int64_t a_cs,
                                     int64_t a_bs, const void* b, int64_t b_rs,
                                     int64_t b_cs, int64_t b_bs, int ab_dtype,
