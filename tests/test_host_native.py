@@ -45,6 +45,38 @@ def test_errors_stay_errors(mojo):
     assert m.view(4, 6, 1, 1, 1, 1, 1, 1).unsqueeze(0).dim() == 9  # a view has no allocation's limit
 
 
+@pytest.mark.parametrize("shape,dtype", [
+    ((2 ** 61,), torch.float32),  # 2^63 bytes: negative
+    ((2 ** 30, 2 ** 31), torch.float32),
+    ((2 ** 62,), torch.float32),  # 2^64 bytes: zero
+    ((2 ** 62 + 4,), torch.float32),  # a small positive number
+    ((2 ** 62,), torch.bfloat16), ((2 ** 63 - 1,), torch.bfloat16), ((2 ** 63 - 1,), torch.int64),
+    ((2 ** 32, 2 ** 32), torch.uint8), ((2 ** 32, 2 ** 32, 3), torch.float32), ((2 ** 21,) * 8, torch.uint8),
+])
+def test_sizes_past_64_bits_are_refused(mojo, shape, dtype):
+    """Counts of elements or bytes that do not fit in 64 bits, whatever they
+    wrap to, raise (as torch.empty does for the CPU) and allocate nothing."""
+    for make in (lambda: torch.empty(shape, dtype=dtype, device="mojo"), lambda: torch.zeros(shape, dtype=dtype, device="mojo"),
+                 lambda: TorchMojoTensor._alloc(shape, dtype, 0), lambda: host().alloc(shape, dtype, 0)):
+        with pytest.raises(Exception):  # noqa: B017 torch's own checks and this module's
+            make()
+    one = torch.zeros((1,) * len(shape), dtype=dtype).to("mojo")
+    with pytest.raises(Exception):  # noqa: B017
+        one.expand(shape).contiguous()
+
+
+def test_views_past_64_bits_are_refused(mojo):
+    empty, m = torch.zeros(0, 4).to("mojo"), torch.zeros(4, 6).to("mojo")
+    for call in (lambda: empty.view(2 ** 32, 2 ** 32), lambda: m.view(2 ** 32, 2 ** 32, 24), lambda: empty.view(2 ** 33, 2 ** 33, 0),
+                 lambda: m.expand(2 ** 40, 2 ** 40, 4, 6), lambda: torch.as_strided(m, (1,), (1,), 2 ** 62),
+                 lambda: host().view_of(m, (2 ** 32, 2 ** 32), (0, 0), 0, None), lambda: host().narrow(m, 0, 2 ** 62, 2 ** 62),
+                 lambda: host().view_of(m[1:], (1,), (1,), -2 ** 63, None),
+                 lambda: host().make(m._holder, m._ptr, (2 ** 32, 2 ** 32), (0, 0), 0, m.dtype, 0, None)):
+        with pytest.raises((RuntimeError, IndexError)):
+            call()
+    assert empty.view(2 ** 40, 0).shape == (2 ** 40, 0) and m.expand(2 ** 40, 4, 6).shape[0] == 2 ** 40
+
+
 @pytest.fixture(scope="module")
 def both():
     return ek._load(), ek._NativeLibrary(ek._load())

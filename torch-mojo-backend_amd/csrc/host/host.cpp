@@ -338,28 +338,48 @@ PyObject* tuple_of(const int64_t* v, int n) {
   return t;
 }
 
-int64_t product(const int64_t* v, int n) {
-  int64_t p = 1;
-  for (int i = 0; i < n; ++i) p *= v[i];
-  return p;
+// Sizes are Python integers, so a count of elements or bytes may not fit in 64
+// bits: then it is refused, as torch refuses it.
+bool overflow(const char* what) {
+  PyErr_Format(PyExc_RuntimeError, "%s overflows 64 bits", what);
+  return false;
+}
+
+// The element count of a shape; false with an exception when it does not fit.
+bool product(const int64_t* v, int n, int64_t* p) {
+  bool over = false;
+  *p = 1;
+  for (int i = 0; i < n; ++i) {
+    if (v[i] == 0) {
+      *p = 0;
+      return true;
+    }
+    over |= __builtin_mul_overflow(*p, v[i], p);
+  }
+  return !over || overflow("the number of elements");
 }
 
 bool contiguous(const int64_t* shape, const int64_t* strides, int n) {
   int64_t expected = 1;
+  bool over = false;
   for (int i = n - 1; i >= 0; --i) {
     if (shape[i] == 1) continue;
-    if (strides[i] != expected) return false;
-    expected *= shape[i];
+    if (over || strides[i] != expected) return false;
+    over = __builtin_mul_overflow(expected, shape[i], &expected);
   }
   return true;
 }
 
-void row_major(const int64_t* shape, int n, int64_t* strides) {
+// False with an exception when a stride does not fit.
+bool row_major(const int64_t* shape, int n, int64_t* strides) {
   int64_t acc = 1;
+  bool over = false;
   for (int i = n - 1; i >= 0; --i) {
+    if (over) return overflow("a stride");
     strides[i] = acc;
-    acc *= shape[i] > 1 ? shape[i] : 1;
+    over = __builtin_mul_overflow(acc, shape[i] > 1 ? shape[i] : 1, &acc);
   }
+  return true;
 }
 
 // make(holder, ptr, shape, strides, offset, dtype, device, contiguous | None)
@@ -374,9 +394,11 @@ PyObject* make(PyObject*, PyObject* const* a, Py_ssize_t n) {
     if (!PyErr_Occurred()) PyErr_SetString(PyExc_ValueError, "shape and strides differ in length");
     return nullptr;
   }
+  int64_t numel;
+  if (!product(shape, nd, &numel)) return nullptr;
   const bool c = a[7] == Py_None ? contiguous(shape, strides, nd) : PyObject_IsTrue(a[7]) == 1;
   PyObject *sh = tuple_of(shape, nd), *st = tuple_of(strides, nd), *t = nullptr;
-  if (sh && st) t = make_impl(a[0], a[1], sh, st, a[4], a[5], a[6], product(shape, nd), c);
+  if (sh && st) t = make_impl(a[0], a[1], sh, st, a[4], a[5], a[6], numel, c);
   Py_XDECREF(sh), Py_XDECREF(st);
   return t;
 }
@@ -419,10 +441,13 @@ PyObject* alloc_impl(const int64_t* shape, int nd, PyObject* dtype, PyObject* de
     if (!PyErr_Occurred()) PyErr_Format(PyExc_TypeError, "unsupported dtype %R", dtype);
     return nullptr;
   }
-  int64_t strides[kMaxRank];
-  row_major(shape, nd, strides);
-  const int64_t numel = product(shape, nd);
-  PyObject* holder = alloc_bytes(numel * PyLong_AsLongLong(itemsize), device);
+  int64_t strides[kMaxRank], numel, bytes;
+  if (!product(shape, nd, &numel) || !row_major(shape, nd, strides)) return nullptr;
+  if (__builtin_mul_overflow(numel, (int64_t)PyLong_AsLongLong(itemsize), &bytes)) {
+    overflow("the number of bytes");
+    return nullptr;
+  }
+  PyObject* holder = alloc_bytes(bytes, device);
   if (!holder) return nullptr;
   PyObject *t = nullptr, *ptr = PyObject_CallMethodNoArgs(holder, s_data_ptr);
   PyObject *sh = tuple_of(shape, nd), *st = tuple_of(strides, nd), *zero = PyLong_FromLong(0);
@@ -474,22 +499,29 @@ bool read(PyObject* t, Meta* m) {
   m->nd = ints_of(shape, m->shape);
   if (m->nd < 0 || ints_of(strides, m->strides) != m->nd) return false;
   m->contig = contig == Py_True;
-  m->numel = product(m->shape, m->nd);
-  return true;
+  return product(m->shape, m->nd, &m->numel);
 }
 
 // A view of m with another shape and strides, `delta` elements further on.
 PyObject* view_impl(const Meta& m, const int64_t* shape, const int64_t* strides, int nd, int64_t delta, bool contig) {
+  int64_t numel;
+  if (!product(shape, nd, &numel)) return nullptr;
   PyObject *t = nullptr, *sh = tuple_of(shape, nd), *st = tuple_of(strides, nd);
   PyObject *ptr = m.ptr, *off = m.offset;
   if (delta) {
-    const int64_t p = PyLong_AsLongLong(m.ptr), o = PyLong_AsLongLong(m.offset), e = PyLong_AsLongLong(m.itemsize);
-    ptr = PyLong_FromLongLong(p + delta * e);
-    off = PyLong_FromLongLong(o + delta);
+    int64_t p = PyLong_AsLongLong(m.ptr), o = PyLong_AsLongLong(m.offset), by = PyLong_AsLongLong(m.itemsize);
+    ptr = off = nullptr;
+    if (__builtin_mul_overflow(delta, by, &by) || __builtin_add_overflow(p, by, &p) ||
+        __builtin_add_overflow(o, delta, &o)) {
+      overflow("the address of a view");
+    } else {
+      ptr = PyLong_FromLongLong(p);
+      off = PyLong_FromLongLong(o);
+    }
   } else {
     Py_INCREF(ptr), Py_INCREF(off);
   }
-  if (sh && st && ptr && off) t = make_impl(m.holder, ptr, sh, st, off, m.dtype, m.device, product(shape, nd), contig);
+  if (sh && st && ptr && off) t = make_impl(m.holder, ptr, sh, st, off, m.dtype, m.device, numel, contig);
   Py_XDECREF(sh), Py_XDECREF(st), Py_XDECREF(ptr), Py_XDECREF(off);
   return t;
 }
@@ -513,9 +545,13 @@ PyObject* view_of(PyObject*, PyObject* const* a, Py_ssize_t n) {
     if (!PyErr_Occurred()) PyErr_SetString(PyExc_ValueError, "shape and strides differ in length");
     return nullptr;
   }
-  const int64_t base = PyLong_AsLongLong(m.offset);
+  int64_t delta;
+  if (__builtin_sub_overflow(off, (int64_t)PyLong_AsLongLong(m.offset), &delta)) {
+    overflow("the offset of a view");
+    return nullptr;
+  }
   const bool c = a[4] == Py_None ? contiguous(shape, strides, nd) : PyObject_IsTrue(a[4]) == 1;
-  return view_impl(m, shape, strides, nd, off - base, c);
+  return view_impl(m, shape, strides, nd, delta, c);
 }
 
 // alias(t)
@@ -560,12 +596,14 @@ PyObject* narrow(PyObject*, PyObject* const* a, Py_ssize_t n) {
   }
   if (!read(a[0], &m)) return not_mojo();
   if (!as_i64(a[1], &d) || !as_i64(a[2], &start) || !as_i64(a[3], &len)) return nullptr;
-  if (d < 0 || d >= m.nd || start < 0 || len < 0 || start + len > m.shape[d]) {
+  int64_t delta = 0;
+  if (d < 0 || d >= m.nd || start < 0 || len < 0 || start > m.shape[d] || len > m.shape[d] - start ||
+      __builtin_mul_overflow(start, m.strides[d], &delta)) {
     PyErr_SetString(PyExc_IndexError, "narrow: out of range");
     return nullptr;
   }
   m.shape[d] = len;
-  return view_impl(m, m.shape, m.strides, m.nd, start * m.strides[d], contiguous(m.shape, m.strides, m.nd));
+  return view_impl(m, m.shape, m.strides, m.nd, delta, contiguous(m.shape, m.strides, m.nd));
 }
 
 // reshape_contiguous(t, size): the view of a contiguous tensor, or None when
@@ -585,8 +623,7 @@ PyObject* reshape_contiguous(PyObject*, PyObject* const* a, Py_ssize_t n) {
   int64_t known = 1;
   for (int i = 0; i < nd; ++i) {
     if (shape[i] == -1 && unknown < 0) unknown = i;
-    else if (shape[i] < 0) Py_RETURN_NONE;
-    else known *= shape[i];
+    else if (shape[i] < 0 || __builtin_mul_overflow(known, shape[i], &known)) Py_RETURN_NONE;
   }
   if (unknown >= 0) {
     if (known == 0 || m.numel % known) Py_RETURN_NONE;
@@ -594,7 +631,7 @@ PyObject* reshape_contiguous(PyObject*, PyObject* const* a, Py_ssize_t n) {
   } else if (known != m.numel) {
     Py_RETURN_NONE;
   }
-  row_major(shape, nd, strides);
+  if (!row_major(shape, nd, strides)) return nullptr;
   return view_impl(m, shape, strides, nd, 0, true);
 }
 
