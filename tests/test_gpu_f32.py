@@ -114,6 +114,28 @@ def test_attention_f32_matrix_cores(kernels, d, causal, sq, skv, layout):
         assert bool((err <= bound).all()), (name, float((err / bound.clamp_min(1e-300)).max()))
 
 
+@pytest.mark.parametrize("d", [32, 64, 128])
+def test_attention_f32_scores_are_partial_sums(kernels, d):
+    """A score's rounding error is that of eight partial sums (four at head_dim
+    32) added in a tree, not of one chain.  With one key LSE is the score; its
+    terms are positive, so a rounding of a partial sum that holds a share x of
+    the score is off by at most u x (u = 2^-24; by u x / sqrt(3) in the root
+    mean square).  Partial sums of d / 8 terms and the tree have shares whose
+    squares sum to 2.4 (the factor to natural logarithms adds 1, the operand's
+    scaling next to nothing): 1.1 u.  One chain of d terms has d / 3 more, 1.9 u
+    (d = 32) to 3.8 u."""
+    n = 8192
+    gen = torch.Generator().manual_seed(d)
+    q, k = 1 + torch.rand(1, 1, n, d, generator=gen), 1 + torch.rand(1, 1, 1, d, generator=gen)
+    tq, tk, o, lse = dev(q), dev(k), torch.empty(1, 1, n, d, device="cuda"), torch.empty(1, 1, n, device="cuda")
+    call("mi355x_attn_fwd_gen", p(o), bhs(o), p(lse), p(tq), bhs(tq), p(tk), bhs(tk), p(tk), bhs(tk), 1, 1, 1, n, 1, d, 1.0,
+         0, 0, 0, None)
+    log2e, ln2 = (torch.tensor(x, dtype=torch.float64).float().double() for x in (1.4426950408889634, 0.6931471805599453))
+    exact = (q.double() * k.double()).sum(-1) * (log2e * ln2)
+    rms = float(((host(lse).double() - exact) / exact).square().mean().sqrt()) * 2.0 ** 24
+    assert rms <= 1.1, rms
+
+
 def test_attention_f32_infinities_and_nan(kernels, mojo):
     """A NaN or infinite element shows where it shows on the CPU: in its own
     query's row, and in every later query's through its key."""

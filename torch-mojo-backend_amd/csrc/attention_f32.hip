@@ -20,9 +20,9 @@
 // enough blocks, and the operand reads are still a quarter of the LDS rate.
 //
 // Causal, against the element-per-lane kernels that took these calls:
-// [4, 12, 255, 64] forward 108 -> 18.7 us, dK, dV and dQ 246 -> 40 us;
-// [8, 12, 512, 64] 429 -> 69 us and 1053 -> 184 us (47 TFLOP/s both ways,
-// counting the causal half).
+// [4, 12, 255, 64] forward 105 -> 18.1 us, backward 243 -> 43.2 us; [8, 12, 512,
+// 64] 424 -> 70.4 us and 1033 -> 183 us (46 and 44 TFLOP/s, counting the causal
+// half).
 #include <math.h>
 
 #include "attention_f32.h"
@@ -122,20 +122,35 @@ __device__ __forceinline__ void block_of(uint32_t L, uint32_t total, uint32_t pe
   *x = i - *bh * per_head;
 }
 
-// s[sub] (16 keys x 16 queries, C layout) += rows of the tile times the
-// register fragments q of the wave's 16 columns.
+// s[sub] (16 keys x 16 queries, C layout) = rows of the tile times the
+// register fragments q of the wave's 16 columns.  A score is the sum of eight
+// partial chains of D / 8 terms (four of 8 at D = 32), added in a tree, as in
+// the element-per-lane kernels.  One chain of D terms was further from 64 bits
+// than those (2-norm error of O at [4, 4, 64, 128], full: 2.3e-7 there, 3.6e-7
+// in one chain, 1.9e-7 in eight; of dQ at [4, 12, 255, 64], causal: 3.4e-7,
+// 3.9e-7, 3.2e-7).  The adds take about 5% of the kernels' time ([4, 12, 255,
+// 64] forward 17.2 -> 18.1 us, backward 40.7 -> 43.2); four chains 3%, but
+// there short sequences stayed up to 2% further off.
 template <int D>
 __device__ __forceinline__ void scores(const char* t, const f32x4 (&q)[D / 16], int lr, int lg, f32x4 (&s)[2]) {
+  constexpr int N = D >= 64 ? 8 : 4;  // chains
 #pragma unroll
-  for (int ks = 0; ks < D / 16; ++ks) {
-    const f32x4 a0 = Tile<D>::row(t, lr, ks, lg), a1 = Tile<D>::row(t, 16 + lr, ks, lg);
+  for (int sub = 0; sub < 2; ++sub) {
+    f32x4 c[N];
 #pragma unroll
-    for (int j = 0; j < 4; ++j) {
-      s[0] = mma(a0[j], q[ks][j], s[0]);
-      s[1] = mma(a1[j], q[ks][j], s[1]);
+    for (int i = 0; i < N; ++i) c[i] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int ks = 0; ks < D / 16; ++ks) {
+      const f32x4 a = Tile<D>::row(t, sub * 16 + lr, ks, lg);
+#pragma unroll
+      for (int j = 0; j < 4; ++j) c[(ks * 4 + j) % N] = mma(a[j], q[ks][j], c[(ks * 4 + j) % N]);
     }
+#pragma unroll
+    for (int w = N / 2; w > 0; w /= 2)
+#pragma unroll
+      for (int i = 0; i < w; ++i) c[i] += c[i + w];
+    s[sub] = c[0];
   }
-  settle(s);
 }
 
 // acc[f] (head-dim fragment f x 16 columns) += tile^T p
@@ -203,7 +218,7 @@ __global__ void __launch_bounds__(kNT, 2) fwd_f32(AttnF32 p, uint32_t nblk) {
     }
     if (k0 >= wend) continue;
     const char* kt = lds + cur * 2 * T::BYTES;
-    f32x4 s[2] = {f32x4{0.f, 0.f, 0.f, 0.f}, f32x4{0.f, 0.f, 0.f, 0.f}};
+    f32x4 s[2];
     scores<D>(kt, q, lr, lg, s);
     if (k0 + kRow > p.Skv || (p.causal && k0 + kRow - 1 > w0)) {
 #pragma unroll
@@ -296,7 +311,7 @@ __device__ __forceinline__ void dq_f32(const AttnF32& p, uint32_t L, uint32_t to
     }
     if (k0 >= wend) continue;
     const char* kt = lds + cur * 2 * T::BYTES;
-    f32x4 s[2] = {f32x4{0.f, 0.f, 0.f, 0.f}, f32x4{0.f, 0.f, 0.f, 0.f}}, dp[2] = {s[0], s[1]};
+    f32x4 s[2], dp[2];
     scores<D>(kt, q, lr, lg, s);
     scores<D>(kt + T::BYTES, dO, lr, lg, dp);
     const bool masked = k0 + kRow > p.Skv || (p.causal && k0 + kRow - 1 > w0);
@@ -348,7 +363,7 @@ __device__ __forceinline__ void dkv_f32(const AttnF32& p, uint32_t L, uint32_t t
     if (r0 + kRow < p.Sq) issue(r0 + kRow, cur ^ 1);
     if (p.causal && r0 + kRow - 1 < w0) continue;  // no query of the tile sees this wave's keys
     const char* qt = lds + cur * 2 * T::BYTES;
-    f32x4 s[2] = {f32x4{0.f, 0.f, 0.f, 0.f}, f32x4{0.f, 0.f, 0.f, 0.f}}, dp[2] = {s[0], s[1]};
+    f32x4 s[2], dp[2];
     scores<D>(qt, k, lr, lg, s);
     scores<D>(qt + T::BYTES, v, lr, lg, dp);
     const bool masked = r0 + kRow > p.Sq || (p.causal && r0 < w0 + 15);
