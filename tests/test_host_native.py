@@ -103,6 +103,18 @@ def test_calls_match_ctypes(both):
             n.mi355x_attn_fwd(*wrong)
 
 
+@pytest.mark.parametrize("m,n,k,tile,splits", [(768, 768, 4096, 64, 3), (768, 768, 8192, 128, 13), (384, 1536, 8192, 128, 13),
+                                               (512, 2048, 4096, 128, 8), (2304, 768, 2048, 64, 1), (256, 1152, 16384, 128, 26)])
+def test_weight_gradient_plans(both, m, n, k, tile, splits):
+    """The K splits (and, by the row sums' slots, the tiles) that weight gradients
+    dY^T X take, from the workspace they ask for: 64x64 tiles up to 3.8e9
+    multiply-adds, 128x128 above."""
+    up = lambda v: (v + 255) // 256 * 256  # noqa: E731
+    got = both[1].mi355x_gemm_workspace_bytes(4096, 1, m, 0, 8192, n, 1, 0, 1, 1, m, n, k)
+    slots = -(-n // tile) * 2
+    assert got == (up(splits * m * n * 4) + up(splits * slots * m * 4) if splits > 1 else 0)
+
+
 def test_every_entry_point_is_native(both):
     slow = {name for name in ek.SIGNATURES if getattr(both[1], name).__class__ is not len.__class__}
     assert slow == {"mi355x_abi_version", "mi355x_last_error", "mi355x_target", "mi355x_source_hash"}
