@@ -69,10 +69,13 @@ def test_gemm_stores_at_any_alignment(kernels, m, n, layout, c_dtype, flags):
 
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
 @pytest.mark.parametrize("layout", ["NT", "NN", "TN", "TT"])
-@pytest.mark.parametrize("m,n,k,batch", [(700, 6000, 768, 1), (2500, 10007, 520, 2), (130, 33000, 136, 1)])
+@pytest.mark.parametrize("m,n,k,batch", [(700, 6000, 768, 1), (2500, 10007, 520, 2), (130, 33000, 136, 1), (400, 4104, 640, 2),
+                                         (9000, 15003, 288, 1)])
 def test_gemm_groups_of_tile_rows(kernels, dtype, layout, m, n, k, batch):
     """B beyond 8 MB: the tiles are walked in groups of rows, the last group a
-    partial one.  Each element of C against products exact in f64."""
+    partial one; beyond 4 MB in one group where A is small; and row by row where
+    K is short and C, in rows that are not aligned, past 256 MB.  Each element of
+    C against products exact in f64."""
     gen = torch.Generator().manual_seed(m + n + k)
     A, B = (torch.randn(batch, *s, generator=gen).to(dtype) for s in ((m, k), (k, n)))
     ta = dev((A.transpose(1, 2) if layout[0] == "T" else A).contiguous())

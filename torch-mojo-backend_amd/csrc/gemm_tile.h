@@ -833,16 +833,26 @@ int launch_tile(GemmArgs g, int64_t batch, int splits, hipStream_t s) {
   const int tm = (int)ceil_div(g.m, C::BM), tn = (int)ceil_div(g.n, C::BN);
   g.tiles_n = tn;
   g.batch = (int)batch;
-  // Row by row reads all of B for each tile row: when B is past an XCD's 4 MB
-  // L2, walk as many tile rows together as keep their part of A in half of it
-  // (logits of 50257 columns at K = 768: 2048 rows 238 -> 185 us, 8192 rows 799
-  // -> 764 us, 16384 rows the same).
+  // Row by row reads all of B for each tile row: when B is past two of an
+  // XCD's 4 MB L2, walk as many tile rows together as keep their part of A in
+  // half of it (logits of 50257 columns at K = 768: 2048 rows 230 -> 161 us, 8192
+  // rows 799 -> 764 us, 16384 rows the same).  From one L2 on where that is all
+  // of A: then each XCD reads its part of B once (512 x 4096 at K = 1024 13.1 ->
+  // 9.5 us and with an n-contiguous B 15.9 -> 9.5, 1021 x 3072 at K = 768 13.0 ->
+  // 11.2; with more of A 2048 x 768 at K = 3072 19.6 -> 21.0; two tile rows gain
+  // nothing, 65 x 4096 at K = 640 5.4 -> 5.6).
+  // Not where a short K leaves the stores of C in front, past the 256 MB
+  // Infinity Cache, in rows that are not 16-byte aligned: their lines are
+  // written in parts, which row by row meet in the L2 sooner (16384 x 30001 at
+  // K = 256 / 512 / 640 / 704, us: in groups 539 / 658 / 699 / 691, row by row
+  // 374 / 561 / 653 / 698; 4096 x 30001 at K = 512 146 / 154).
   g.group = 1;
-  const int64_t panel = (int64_t)C::BM * min(g.k, g.kchunk) * (int64_t)sizeof(T);
-  if (g.n * min(g.k, g.kchunk) * (int64_t)sizeof(T) > (8 << 20)) {
-    const int64_t rows = (2 << 20) / panel;
+  const int64_t k = min(g.k, g.kchunk), b_bytes = g.n * k * (int64_t)sizeof(T);
+  const int64_t c_es = g.c_dt == MI355X_F32 ? 4 : 2, rows = (2 << 20) / (C::BM * k * (int64_t)sizeof(T));
+  const bool c_parts = !g.part && (g.c_rs * c_es % 16 != 0 || (uintptr_t)g.c % 16 != 0) &&
+                       g.m * g.n * c_es > (256 << 20) && k < 704;
+  if (!c_parts && (b_bytes > (8 << 20) || (b_bytes > (4 << 20) && tm > 2 && tm <= rows)))
     g.group = (int)(rows < 1 ? 1 : rows > tm ? tm : rows);
-  }
   dim3 grid((unsigned)(tm * tn), (unsigned)(batch * splits));
   if constexpr (CFG != 3) {  // which has no row sums
     if (g.rowsum) return launch_layout<T, CFG, KT, true>(g, grid, s);
