@@ -16,7 +16,8 @@ def _copy(dst, src):
 
 
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32, torch.uint8, torch.int64])
-@pytest.mark.parametrize("shape", [(3, 5, 7, 64), (2, 1, 9, 16), (4, 3, 2, 520), (2, 3, 4, 5), (1, 6, 1, 8)])
+@pytest.mark.parametrize("shape", [(3, 5, 7, 64), (2, 1, 9, 16), (4, 3, 2, 520), (2, 3, 4, 5), (1, 6, 1, 8),
+                                   (2, 70, 3, 131), (65, 8, 64, 9), (130, 7, 2, 66)])
 def test_copy_every_order(kernels, dtype, shape):
     """Source and destination each in every dimension order, dense or as a
     slice of a wider buffer, on bases that are 16-byte aligned and not."""
@@ -38,3 +39,17 @@ def test_copy_every_order(kernels, dtype, shape):
         torch.as_strided(want, dst.shape, dst.stride(), dst.storage_offset()).copy_(src)
         _copy(dst, src)
         assert torch.equal(store, want), (ps, pd, off, wide)
+
+
+@pytest.mark.parametrize("src_dtype,dst_dtype", [(torch.float32, torch.bfloat16), (torch.float32, torch.float16),
+                                                 (torch.bfloat16, torch.float32), (torch.float16, torch.float32),
+                                                 (torch.int64, torch.float32), (torch.bfloat16, torch.float16)])
+@pytest.mark.parametrize("shape", [(3, 70, 131), (129, 8, 64), (5, 7, 300)])
+def test_cast_every_order(kernels, src_dtype, dst_dtype, shape):
+    """Casts between every pair of dimension orders: the rounding of torch's."""
+    values = torch.randn(torch.Size(shape).numel(), device="cuda") * 100
+    for ps, pd in itertools.product(itertools.permutations(range(3)), repeat=2):
+        src = values.to(src_dtype).view([shape[i] for i in ps]).permute([ps.index(i) for i in range(3)])
+        dst = torch.zeros([shape[i] for i in pd], dtype=dst_dtype, device="cuda").permute([pd.index(i) for i in range(3)])
+        _copy(dst, src)
+        assert torch.equal(dst, src.to(dst_dtype)), (ps, pd)

@@ -510,6 +510,56 @@ __global__ void __launch_bounds__(kThreads) copy_outer_b128(uint8_t* __restrict_
   }
 }
 
+// Copies whose unit strides lie in different dimensions (d of the destination,
+// s of the source): 64 x 64 tiles of the two go through LDS, so that the reads
+// are rows of s and the writes rows of d.  HBM-bound.  Element by element no
+// order of the dimensions serves both sides: 3000 x 200 x 40 elements of 4
+// bytes, the source in the order 0, 2, 1, the destination in 1, 0, 2, took 163
+// us in the caller's order and 415 in the destination's, 1000 x 50257 transposed
+// 736 and 341; in tiles 46 and 138.  An s shorter than 16 leaves most of a
+// wave's lanes without a read (8 x 1024 x 12 x 64 elements of 4 bytes, s = 8: 37
+// us element by element, 58 in tiles).
+struct TwoUnit {
+  int64_t nd, ns;              // extents of d and s
+  int64_t dst_s, src_d;        // the other operand's stride along each
+  int64_t tiles_s, tiles_d, tiles;
+  int nouter;                  // the remaining dimensions
+  int64_t shape[MI355X_MAX_RANK], dst[MI355X_MAX_RANK], src[MI355X_MAX_RANK];
+};
+template <typename TI, typename TO>
+__device__ __forceinline__ TO cast_elem(TI v) {
+  if constexpr (std::is_same<TI, TO>::value) return v;
+  else return from_f32<TO>(to_f32(v));
+}
+template <typename TI, typename TO>
+__global__ void __launch_bounds__(kThreads) copy_tiles(TO* __restrict__ dst, const TI* __restrict__ src, TwoUnit g) {
+  __shared__ TI tile[64][65];
+  const int x = threadIdx.x & 63, y = threadIdx.x >> 6;
+  for (int64_t t = blockIdx.x; t < g.tiles; t += gridDim.x) {
+    int64_t r = t / g.tiles_s, sb = 0, db = 0;
+    const int64_t s0 = (t - r * g.tiles_s) * 64, q = r / g.tiles_d, d0 = (r - q * g.tiles_d) * 64;
+    r = q;
+    for (int i = g.nouter - 1; i >= 0; --i) {
+      const int64_t n = r / g.shape[i], c = r - n * g.shape[i];
+      sb += c * g.src[i], db += c * g.dst[i];
+      r = n;
+    }
+    const int ns = (int)min((int64_t)64, g.ns - s0), nd = (int)min((int64_t)64, g.nd - d0);
+    const TI* S = src + sb + d0 * g.src_d + s0;
+    TO* D = dst + db + s0 * g.dst_s + d0;
+    if (x < ns)
+#pragma unroll
+      for (int j = 0; j < 64; j += 4)
+        if (j + y < nd) tile[j + y][x] = S[(j + y) * g.src_d + x];
+    __syncthreads();
+    if (x < nd)
+#pragma unroll
+      for (int j = 0; j < 64; j += 4)
+        if (j + y < ns) D[(j + y) * g.dst_s + x] = cast_elem<TI, TO>(tile[x][j + y]);
+    __syncthreads();
+  }
+}
+
 // Dense same-dtype copy, 16 bytes per thread-iteration.
 __global__ void __launch_bounds__(kThreads) copy_b128(uint4* __restrict__ out,
                                                       const uint4* __restrict__ in, int64_t n16) {
@@ -565,6 +615,61 @@ int launch_map(const MapArgs& a, const Geo& g, int64_t n, int kind, hipStream_t 
 }
 
 bool valid_dtype(int dt) { return dt >= MI355X_F32 && dt <= MI355X_BOOL; }
+
+template <typename TI, typename TO>
+int launch_tiles(void* dst, const void* src, const TwoUnit& t, hipStream_t s) {
+  copy_tiles<TI, TO><<<(unsigned)min(t.tiles, (int64_t)65536), kThreads, 0, s>>>((TO*)dst, (const TI*)src, t);
+  return check_launch("mi355x_copy");
+}
+
+// copy_tiles on a geometry in the destination's order (operand 0): -1 when it
+// does not take the copy (one dimension is contiguous on both sides, too short a
+// one, a cast of other types).
+int copy_two_unit(void* dst, int dst_dt, const void* src, int src_dt, const Geo& g, hipStream_t s) {
+  const int d = g.ndim - 1;
+  int c = -1;
+  for (int i = 0; i < d; ++i)
+    if (g.st[1][i] == 1) c = i;
+  if (c < 0 || g.st[0][d] != 1 || g.st[1][d] == 1 || g.shape[d] < 8 || g.shape[c] < 16) return -1;
+  TwoUnit t{};
+  t.nd = g.shape[d], t.ns = g.shape[c], t.dst_s = g.st[0][c], t.src_d = g.st[1][d];
+  t.tiles_s = (t.ns + 63) / 64, t.tiles_d = (t.nd + 63) / 64, t.tiles = t.tiles_s * t.tiles_d;
+  for (int i = 0; i < d; ++i) {
+    if (i == c) continue;
+    t.shape[t.nouter] = g.shape[i], t.dst[t.nouter] = g.st[0][i], t.src[t.nouter] = g.st[1][i];
+    ++t.nouter;
+    t.tiles *= g.shape[i];
+  }
+  if (dst_dt == src_dt) switch (dtype_size(dst_dt)) {
+      case 1: return launch_tiles<uint8_t, uint8_t>(dst, src, t, s);
+      case 2: return launch_tiles<uint16_t, uint16_t>(dst, src, t, s);
+      case 4: return launch_tiles<uint32_t, uint32_t>(dst, src, t, s);
+      default: return launch_tiles<uint64_t, uint64_t>(dst, src, t, s);
+    }
+#define CAST(DI, TI, DO, TO) \
+  if (src_dt == DI && dst_dt == DO) return launch_tiles<TI, TO>(dst, src, t, s);
+  CAST(MI355X_F32, float, MI355X_BF16, bf16)
+  CAST(MI355X_F32, float, MI355X_F16, f16)
+  CAST(MI355X_BF16, bf16, MI355X_F32, float)
+  CAST(MI355X_F16, f16, MI355X_F32, float)
+#undef CAST
+  return -1;
+}
+
+// How far apart in a walk of g's dimensions neighbours in memory come, for the
+// operand where they come furthest apart.
+int64_t reach(const Geo& g) {
+  int64_t most = 1;
+  for (int j = 0; j < g.nops; ++j) {
+    int at = g.ndim - 1;
+    for (int i = at - 1; i >= 0; --i)
+      if (g.st[j][i] < g.st[j][at]) at = i;
+    int64_t n = 1;
+    for (int i = at + 1; i < g.ndim; ++i) n *= g.shape[i];
+    if (n > most) most = n;
+  }
+  return most;
+}
 
 inline bool aligned(const void* p, size_t a) { return ((uintptr_t)p % a) == 0; }
 
@@ -627,15 +732,16 @@ extern "C" int mi355x_copy(void* dst, int dst_dtype, const int64_t* dst_strides,
     const int64_t es = (int64_t)dtype_size(dst_dtype), rb = g.shape[in] * es;
     bool wide = rb % 16 == 0 && aligned(dst, 16) && aligned(src, 16);
     for (int d = 0; d < in; ++d) wide = wide && (g.st[0][d] * es) % 16 == 0 && (g.st[1][d] * es) % 16 == 0;
-    if (wide && g.ndim == 2 && rb >= 1024) {
+    const int64_t chunks = n * es / 16;
+    const bool few = chunks < (int64_t)1 << 31;  // 32-bit index and grid stride
+    if (wide && g.ndim == 2 && (rb >= 1024 || !few)) {
       int64_t blocks = (g.shape[0] + 3) / 4;
       if (blocks > 65536) blocks = 65536;
       copy_rows_b128<<<(unsigned)blocks, kThreads, 0, s>>>((uint8_t*)dst, g.st[0][0] * es, (const uint8_t*)src,
                                                             g.st[1][0] * es, g.shape[0], rb);
       return check_launch("mi355x_copy");
     }
-    const int64_t chunks = n * es / 16;
-    if (wide && chunks < (int64_t)1 << 31) {  // 32-bit index and grid stride
+    if (wide && few) {
       OuterRows o{1, 1, (uint32_t)(rb / 16), {0, 0, 0}, {0, 0, 0}};
       for (int d = 0; d < in; ++d) {
         const int at = 3 - in + d;
@@ -647,6 +753,19 @@ extern "C" int mi355x_copy(void* dst, int dst_dtype, const int64_t* dst_strides,
                                                                (uint32_t)chunks);
       return check_launch("mi355x_copy");
     }
+  }
+  if (g.ndim >= 2) {
+    rc = copy_two_unit(dst, dst_dtype, src, src_dtype, g, s);
+    if (rc >= 0) return rc;
+    // element by element: in the caller's order where the destination's takes
+    // neighbours out of the caches' reach (64 x 12 x 256 x 64 elements of 8 bytes,
+    // a source in the order 0, 3, 2, 1, us: 97, in the destination's order 1, 0,
+    // 2, 3 155; but 77 x 12 x 64 of 4 bytes from 0, 2, 1 to 1, 0, 2 7.9 and 6.7)
+    const int64_t* own[2] = {dst_strides, src_strides};
+    Geo c;
+    rc = build_geo(c, 2, own, shape, ndim, &n);
+    if (rc) return rc;
+    if (reach(g) > (1 << 16) && reach(c) < reach(g)) g = c;
   }
   MapArgs a{};
   a.op = MI355X_OP_IDENTITY;
