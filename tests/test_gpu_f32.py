@@ -136,6 +136,26 @@ def test_attention_f32_scores_are_partial_sums(kernels, d):
     assert rms <= 1.1, rms
 
 
+@pytest.mark.parametrize("d", [32, 64, 128])
+@pytest.mark.parametrize("sq,skv,causal", [(1, 1, 1), (3, 1, 0), (40, 200, 1), (70, 70, 1)])
+def test_attention_f32_one_key_has_no_gradient(kernels, d, sq, skv, causal):
+    """A query that sees one key gives it all its weight, whatever Q and K are: its
+    output is that key's V and its dQ exactly zero (D is summed as dP is), and so is
+    dK where no query sees two keys."""
+    B, H = 2, 3
+    gen = torch.Generator().manual_seed(d + sq)
+    q, do, k, v = (dev(torch.randn(B, H, n, d, generator=gen)) for n in (sq, sq, skv, skv))
+    o, dq, dk, dv, lse = (torch.full_like(x, float("nan")) for x in (q, q, k, v, q[..., 0]))
+    call("mi355x_attn_fwd_gen", p(o), bhs(o), p(lse), p(q), bhs(q), p(k), bhs(k), p(v), bhs(v), B, H, H, sq, skv, d, d ** -0.5,
+         causal, 0, 0, None)
+    ws_n = lib().mi355x_attn_bwd_gen_workspace_bytes(B, H, H, sq, skv, d)
+    call("mi355x_attn_bwd_gen", p(dq), bhs(dq), p(dk), bhs(dk), p(dv), bhs(dv), p(do), bhs(do), p(q), bhs(q), p(k), bhs(k),
+         p(v), bhs(v), p(o), bhs(o), p(lse), B, H, H, sq, skv, d, d ** -0.5, causal, 0, 0, p(workspace(ws_n)), ws_n, None)
+    rows = slice(None) if skv == 1 else slice(1)
+    assert torch.equal(o[:, :, rows], v[:, :, :1].expand_as(o[:, :, rows])) and not dq[:, :, rows].any()
+    assert skv > 1 or not dk.any()
+
+
 def test_attention_f32_infinities_and_nan(kernels, mojo):
     """A NaN or infinite element shows where it shows on the CPU: in its own
     query's row, and in every later query's through its key."""

@@ -132,8 +132,10 @@ __device__ __forceinline__ void block_of(uint32_t L, uint32_t total, uint32_t pe
 // 64] forward 17.2 -> 18.1 us, backward 40.7 -> 43.2); four chains 3%, but
 // there short sequences stayed up to 2% further off.
 template <int D>
+constexpr int kChains = D >= 64 ? 8 : 4;
+template <int D>
 __device__ __forceinline__ void scores(const char* t, const f32x4 (&q)[D / 16], int lr, int lg, f32x4 (&s)[2]) {
-  constexpr int N = D >= 64 ? 8 : 4;  // chains
+  constexpr int N = kChains<D>;
 #pragma unroll
   for (int sub = 0; sub < 2; ++sub) {
     f32x4 c[N];
@@ -257,22 +259,32 @@ __global__ void __launch_bounds__(kNT, 2) fwd_f32(AttnF32 p, uint32_t nblk) {
   if (lg == 0) p.lse[(b * p.H + h) * p.Sq + qi] = l > 0.f ? (m + log2f(l)) * kLn2 : -INFINITY;
 }
 
-// D_i = sum_d dO[i, d] O[i, d]: D / 4 lanes per row, 16 bytes each.
+// D_i = sum_d dO[i, d] O[i, d], in the order of scores(): a lane per partial
+// chain, the terms of an MFMA one after another, then the tree.  Where a query
+// gives all its weight to one key, O is that key's V and dP - D is zero, as it
+// is in exact arithmetic: in another order it is the rounding of both sums
+// (one key: dQ and dK 1e-8 of |dO||V| instead of 0; [1, 2, 3, 64] against 135
+// keys, causal: 2-norm error of dQ 7.1e-7, 3.8e-7 in the element-per-lane kernels).
 template <int D>
 __global__ void __launch_bounds__(kNT) delta_f32(AttnF32 p, int64_t rows) {
-  constexpr int LPR = D / 4;
-  const int64_t row = ((int64_t)blockIdx.x * kNT + threadIdx.x) / LPR;
-  const int c = (threadIdx.x % LPR) * 4;
+  constexpr int N = kChains<D>;
+  const int64_t row = ((int64_t)blockIdx.x * kNT + threadIdx.x) / N;
+  const int c = threadIdx.x % N;
   const bool ok = row < rows;
   float v = 0.f;
   if (ok) {
     const int64_t i = row % p.Sq, bh = row / p.Sq, b = bh / p.H, h = bh % p.H;
-    const f32x4 o = *(const f32x4*)(p.o + b * p.o_b + h * p.o_h + i * p.o_s + c);
-    const f32x4 d = *(const f32x4*)(p.dout + b * p.do_b + h * p.do_h + i * p.do_s + c);
-    v = (o[0] * d[0] + o[1] * d[1]) + (o[2] * d[2] + o[3] * d[3]);
+    const float* o = p.o + b * p.o_b + h * p.o_h + i * p.o_s;
+    const float* d = p.dout + b * p.do_b + h * p.do_h + i * p.do_s;
+#pragma unroll
+    for (int t = 0; t < D / 4; t += N) {
+      const int at = (t + c) / 4 * 16 + (t + c) % 4;
+#pragma unroll
+      for (int g = 0; g < 16; g += 4) v = fmaf(o[at + g], d[at + g], v);
+    }
   }
 #pragma unroll
-  for (int off = LPR / 2; off > 0; off >>= 1) v += __shfl_xor(v, off, 64);
+  for (int off = N / 2; off > 0; off >>= 1) v += __shfl_xor(v, off, 64);
   if (ok && c == 0) p.delta[row] = v;
 }
 
@@ -418,7 +430,7 @@ int run_bwd(const AttnF32& p, hipStream_t s) {
   static const bool ok = opt_in((const void*)bwd_f32<D>, lds_bytes<D>(true));
   if (!ok) return fail(MI355X_ELAUNCH, "mi355x_attn_bwd_gen: cannot reserve %zu bytes of LDS", lds_bytes<D>(true));
   const int64_t rows = p.B * p.H * p.Sq;
-  delta_f32<D><<<ceil_div(rows * (D / 4), kNT), kNT, 0, s>>>(p, rows);
+  delta_f32<D><<<ceil_div(rows * kChains<D>, kNT), kNT, 0, s>>>(p, rows);
   const uint32_t kblk = ceil_div(p.Skv, kBlk), qblk = ceil_div(p.Sq, kBlk);
   const uint32_t heads = (uint32_t)(p.B * p.H);
   bwd_f32<D><<<(kblk + qblk) * heads, kNT, lds_bytes<D>(true), s>>>(p, kblk * heads, kblk, qblk);
