@@ -156,6 +156,25 @@ def test_attention_f32_one_key_has_no_gradient(kernels, d, sq, skv, causal):
     assert skv > 1 or not dk.any()
 
 
+def test_attention_f32_heads_past_one_grid_dimension(kernels):
+    """2^24 blocks of the matrix-core kernels are more threads than one dimension of
+    a launch takes: such calls stay on the general kernels.  With one key O is V, and
+    dV is dO but for the probability, exp2 of a score (8.2 at most) less itself through
+    LSE and back: 4 roundings, u = 2^-24 of 8.2 ln 2 each, and exp2's."""
+    B, H, d = 65535, 257, 32
+    q, k, v, do, o, dq, dk, dv = (torch.empty(B, H, 1, d, device="cuda") for _ in range(8))
+    for x in (q, k, v, do):
+        x.uniform_(-1, 1)
+    lse = torch.empty(B, H, 1, device="cuda")
+    call("mi355x_attn_fwd_gen", p(o), bhs(o), p(lse), p(q), bhs(q), p(k), bhs(k), p(v), bhs(v), B, H, H, 1, 1, d, d ** -0.5,
+         0, 0, 0, None)
+    assert torch.equal(o, v)
+    ws_n = lib().mi355x_attn_bwd_gen_workspace_bytes(B, H, H, 1, 1, d)
+    call("mi355x_attn_bwd_gen", p(dq), bhs(dq), p(dk), bhs(dk), p(dv), bhs(dv), p(do), bhs(do), p(q), bhs(q), p(k), bhs(k),
+         p(v), bhs(v), p(o), bhs(o), p(lse), B, H, H, 1, 1, d, d ** -0.5, 0, 0, 0, p(workspace(ws_n)), ws_n, None)
+    assert bool(((dv - do).abs() <= 26 * 2.0 ** -24 * do.abs()).all()) and not dq.any() and not dk.any()
+
+
 def test_attention_f32_infinities_and_nan(kernels, mojo):
     """A NaN or infinite element shows where it shows on the CPU: in its own
     query's row, and in every later query's through its key."""

@@ -442,8 +442,10 @@ bool wide(const void* p, int64_t b, int64_t h, int64_t s) {
   return ((uintptr_t)p & 15) == 0 && b % 4 == 0 && h % 4 == 0 && s % 4 == 0;
 }
 bool takes(const AttnF32& p) {
-  // 32-bit block counts, and indexes of the delta pass
-  return p.B * p.H * ((p.Sq + p.Skv) / kBlk + 2) < (1ll << 30) && p.B * p.H * p.Sq < (1ll << 33) &&
+  // a launch takes fewer than 2^32 threads in one dimension: bwd_f32's blocks and
+  // delta_f32's chains (the general kernels spread heads and batch over the others)
+  return p.B * p.H * ((p.Sq + kBlk - 1) / kBlk + (p.Skv + kBlk - 1) / kBlk) < (1ll << 24) &&
+         p.B * p.H * p.Sq < (1ll << 29) &&
          wide(p.q, p.q_b, p.q_h, p.q_s) && wide(p.k, p.k_b, p.k_h, p.k_s) && wide(p.v, p.v_b, p.v_h, p.v_s) &&
          wide(p.o, p.o_b, p.o_h, p.o_s);
 }
