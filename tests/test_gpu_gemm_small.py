@@ -139,3 +139,22 @@ def test_gemm_long_k_ends(kernels, layout, k):
     call("mi355x_gemm_ex", p(c), 0, n, 0, *args, 1, None, 0, 0, None, 0, 1, m, n, k, p(ws), ws_n, None)
     a, b = dev(A).double(), dev(B).double()
     assert bool(((c.double() - a @ b).abs() <= (k + 3) * 2.0 ** -23 * (a.abs() @ b.abs())).all())
+
+
+@pytest.mark.parametrize("layout", ["TN", "TT"])
+@pytest.mark.parametrize("k", [72, 520, 1984])
+def test_gemm_row_sums_of_whole_wide_tiles(kernels, layout, k):
+    """Row sums beside the whole K of 256x256 tiles with an m-contiguous A: its
+    fragments are read one at a time there."""
+    m, n = 4090, 4104
+    gen = torch.Generator().manual_seed(k)
+    A, B = (torch.randn(*s, generator=gen).bfloat16() for s in ((4096, k), (k, n)))
+    ta, tb = dev(A.t().contiguous()), dev((B.t() if layout[1] == "T" else B).contiguous())
+    b_rs, b_cs = (n, 1) if layout[1] == "N" else (1, k)
+    args = (p(ta), 1, 4096, 0, p(tb), b_rs, b_cs, 0)
+    ws_n = lib().mi355x_gemm_workspace_bytes(*args, 1, 1, m, n, k)
+    c, sums = torch.full((m, n), float("nan"), device="cuda"), torch.full((m,), float("nan"), device="cuda")
+    call("mi355x_gemm_ex", p(c), 0, n, 0, *args, 1, None, 0, 0, p(sums), 0, 1, m, n, k, p(workspace(ws_n)), ws_n, None)
+    a, b, u = dev(A[:m]).double(), dev(B).double(), (k + 3) * 2.0 ** -23
+    assert bool(((c.double() - a @ b).abs() <= u * (a.abs() @ b.abs())).all())
+    assert bool(((sums.double() - a.sum(1)).abs() <= u * a.abs().sum(1)).all())

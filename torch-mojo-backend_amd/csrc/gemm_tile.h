@@ -688,9 +688,12 @@ __global__ void __launch_bounds__(64 * TileCfg<CFG>::WGM * TileCfg<CFG>::WGN, Ti
       if (RS && ++rs_q == rs_slots) rs_q = 0;
       const int coff = ((ks * 4 + lg) ^ sw) * 16;
       const int64_t kfrag = k0 + ks * 32 + lg * 8;
-      frag bfr[TN], afr[A_K ? 1 : TM];
+      // an m-contiguous A's fragments are read all at once, but one at a time
+      // where the row sums' accumulators leave no registers for them
+      constexpr bool A_ALL = !A_K && !(RS && CFG == 1);
+      frag bfr[TN], afr[A_ALL ? TM : 1];
       if constexpr (!B_K) mn_frags<T, BN, TN>(bt, wn * WN, ks, bfr);
-      if constexpr (!A_K) mn_frags<T, BM, TM>(at, wm * WM, ks, afr);
+      if constexpr (A_ALL) mn_frags<T, BM, TM>(at, wm * WM, ks, afr);
 #pragma unroll
       for (int j = 0; j < TN; ++j) {
         if constexpr (B_K) bfr[j] = *(const frag*)(bt + (wn * WN + j * 16 + lr) * ROWB + coff);
@@ -710,8 +713,9 @@ __global__ void __launch_bounds__(64 * TileCfg<CFG>::WGM * TileCfg<CFG>::WGN, Ti
           lb.template issue_range<KT>(k0 + (S - 1) * BK, nxt + A_BYTES, kend, lo - NA, hi - NA);
         }
         frag af;
-        if constexpr (A_K) af = *(const frag*)(at + (wm * WM + i * 16 + lr) * ROWB + coff);
-        else af = afr[i];
+        if constexpr (A_ALL) af = afr[i];
+        else if constexpr (A_K) af = *(const frag*)(at + (wm * WM + i * 16 + lr) * ROWB + coff);
+        else af = read_frag<T, BM, false>(at, wm * WM + i * 16, ks);
         if (tail) mask_k(af, kfrag, kend);
         if (RS && rs_now) rsum[i] = Mfma<T>::mma(af, ones, rsum[i]);
 #pragma unroll
