@@ -846,16 +846,17 @@ int launch_tile(GemmArgs g, int64_t batch, int splits, hipStream_t s) {
   // 11.2; with more of A 2048 x 768 at K = 3072 19.6 -> 21.0; two tile rows gain
   // nothing, 65 x 4096 at K = 640 5.4 -> 5.6).
   // Not where a short K leaves the stores of C in front, past the 256 MB
-  // Infinity Cache, in rows that are not 16-byte aligned: their lines are
-  // written in parts, which row by row meet in the L2 sooner (16384 x 30001 at
-  // K = 256 / 512 / 640 / 704, us: in groups 539 / 658 / 699 / 691, row by row
-  // 374 / 561 / 653 / 698; 4096 x 30001 at K = 512 146 / 154).
+  // Infinity Cache: in rows that are not 16-byte aligned, whose lines are written
+  // in parts, which row by row meet in the L2 sooner (16384 x 30001 at K = 256 /
+  // 512 / 640 / 704, us: in groups 539 / 658 / 699 / 691, row by row 374 / 561 / 653
+  // / 698; 4096 x 30001 at K = 512 146 / 154); and in one group (5644 x 50257 at K =
+  // 64 295, row by row 268).
   g.group = 1;
   const int64_t k = min(g.k, g.kchunk), b_bytes = g.n * k * (int64_t)sizeof(T);
   const int64_t c_es = g.c_dt == MI355X_F32 ? 4 : 2, rows = (2 << 20) / (C::BM * k * (int64_t)sizeof(T));
-  const bool c_parts = !g.part && (g.c_rs * c_es % 16 != 0 || (uintptr_t)g.c % 16 != 0) &&
-                       g.m * g.n * c_es > (256 << 20) && k < 704;
-  if (!c_parts && (b_bytes > (8 << 20) || (b_bytes > (4 << 20) && tm > 2 && tm <= rows)))
+  const bool c_far = !g.part && g.m * g.n * c_es > (256 << 20);
+  const bool c_parts = (g.c_rs * c_es % 16 != 0 || (uintptr_t)g.c % 16 != 0) && c_far && k < 704;
+  if (!c_parts && (b_bytes > (8 << 20) || (b_bytes > (4 << 20) && !c_far && tm > 2 && tm <= rows)))
     g.group = (int)(rows < 1 ? 1 : rows > tm ? tm : rows);
   dim3 grid((unsigned)(tm * tn), (unsigned)(batch * splits));
   if constexpr (CFG != 3) {  // which has no row sums
