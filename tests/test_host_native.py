@@ -115,6 +115,25 @@ def test_weight_gradient_plans(both, m, n, k, tile, splits):
     assert got == (up(splits * m * n * 4) + up(splits * slots * m * 4) if splits > 1 else 0)
 
 
+def _plan(native, layout, m, n, k):
+    """(tile columns, K splits) of a product, from its workspace: the partial sums
+    and the row sums' slots; splits 1 and no tile without a workspace."""
+    up = lambda v: (v + 255) // 256 * 256  # noqa: E731
+    a = (4096, k, 1, 0) if layout[0] == "N" else (4096, 1, m, 0)
+    b = (8192, n, 1, 0) if layout[1] == "N" else (8192, 1, k, 0)
+    got = native.mi355x_gemm_workspace_bytes(*a, *b, 1, 1, m, n, k)
+    return [(t, s) for t, w in ((64, 2), (128, 2), (192, 2), (256, 4)) for s in range(2, 65)
+            if got == up(s * m * n * 4) + up(s * -(-n // t) * w * m * 4)] if got else [(None, 1)]
+
+
+@pytest.mark.parametrize("layout,m,n,k,tile,splits", [("NT", 80, 768, 3072, 64, 6), ("NT", 568, 1840, 4096, 128, 6),
+                                                      ("NT", 2808, 328, 5144, 128, 7), ("NT", 392, 656, 9192, 64, 6)])
+def test_small_output_plans(both, layout, m, n, k, tile, splits):
+    """From K = 2048 on 64x64 tiles take up to 2.9e9 multiply-adds, counting whole
+    tiles; past that K is split over larger ones."""
+    assert (tile, splits) in _plan(both[1], layout, m, n, k)
+
+
 def test_every_entry_point_is_native(both):
     slow = {name for name in ek.SIGNATURES if getattr(both[1], name).__class__ is not len.__class__}
     assert slow == {"mi355x_abi_version", "mi355x_last_error", "mi355x_target", "mi355x_source_hash"}

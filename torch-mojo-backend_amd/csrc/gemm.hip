@@ -320,17 +320,21 @@ Plan plan_gemm(int64_t batch, int64_t m, int64_t n, int64_t k, bool a_kcontig, b
     }
     planned = true;
   }
-  // Outputs of at most two 64x64 tiles per CU with up to 5e9 multiply-adds (3.8e9
-  // with an m-contiguous A): their larger tiles leave CUs idle and a k-step takes
-  // its latencies, not its MFMA time (us, larger tiles against C64; K = 768 unless
-  // given: 77 x 768 11.6 / 6.3, 255 x 2304 18.1 / 7.5, 512 x 3072 10.6 / 8.0, 1021
-  // x 1024 at K = 1152 20.6 / 9.3, 2048 x 768 10.8 / 7.9; weight gradients 768 x
-  // 768 at K = 4096 24.2 / 19.6, 2304 x 768 at K = 2048 25.1 / 19.5).  Past that
-  // the larger tiles win: more tiles (4096 x 768 11.4 / 12.7, 768 x 3072 at K =
-  // 2048 24.5 / 26.4), or a K long enough to split over all CUs (weight gradients
-  // 1024 x 1024 at K = 4096 26.0 / 27.9, 512 x 2048 at K = 4096 24.3 / 27.8, 768 x
-  // 768 at K = 8192 24.1 / 27.2, at 16384 33.4 / 40.9).
-  if (tiles_of(4, batch, m, n) <= 2 * kCUs && (double)(batch * m * n) * (double)k <= (a_kcontig ? 5e9 : 3.8e9))
+  // Outputs of at most two 64x64 tiles per CU: their larger tiles leave CUs idle
+  // and a k-step takes its latencies, not its MFMA time (us, larger tiles against
+  // C64; K = 768 unless given: 77 x 768 11.6 / 6.3, 255 x 2304 18.1 / 7.5, 512 x
+  // 3072 10.6 / 8.0, 1021 x 1024 at K = 1152 20.6 / 9.3, 2048 x 768 10.8 / 7.9;
+  // weight gradients 768 x 768 at K = 4096 24.2 / 19.6, 2304 x 768 at K = 2048
+  // 25.1 / 19.5).  The larger tiles win where there are more tiles (4096 x 768
+  // 11.4 / 12.7) or a K long enough to split over all CUs: from K = 2048 on past
+  // 2.9e9 multiply-adds, counting whole tiles (264 tiles at K = 5144 27.1 / 34.9,
+  // 171 at 6640 23.9 / 32.0, 294 at 2952 22.1 / 28.6, but 100 at 4096 0.88 of the
+  // time), weight gradients past 3.8e9 (1024 x 1024 at K = 4096 26.0 / 27.9, 512 x
+  // 2048 at K = 4096 24.3 / 27.8, 768 x 768 at K = 8192 24.1 / 27.2, 768 x 3072 at K
+  // = 2048 24.5 / 26.4).
+  const int64_t t64 = tiles_of(4, batch, m, n);
+  const double work64 = (double)t64 * 64 * 64 * (double)k;
+  if (t64 <= 2 * kCUs && (a_kcontig ? k < 2048 || work64 <= 2.9e9 : work64 <= 3.8e9))
     best = Plan{4, 1, k}, planned = false;
   static const char* forced = getenv("MI355X_GEMM_TILE");  // tuning override: "64", "128", "192", "256" or "257" (C256W)
   if (forced) {
