@@ -134,6 +134,14 @@ def test_small_output_plans(both, layout, m, n, k, tile, splits):
     assert (tile, splits) in _plan(both[1], layout, m, n, k)
 
 
+@pytest.mark.parametrize("m,n,k,tile,splits", [(2000, 2248, 2304, None, 1), (3072, 1816, 2304, None, 1),
+                                               (2216, 2280, 4392, 192, 2)])
+def test_splits_of_three_quarters_of_a_round(both, m, n, k, tile, splits):
+    """128x192 tiles on three quarters of the CUs are split where the second block
+    per CU saves more than the partial sums cost."""
+    assert (tile, splits) in _plan(both[1], "NT", m, n, k)
+
+
 def test_every_entry_point_is_native(both):
     slow = {name for name in ek.SIGNATURES if getattr(both[1], name).__class__ is not len.__class__}
     assert slow == {"mi355x_abi_version", "mi355x_last_error", "mi355x_target", "mi355x_source_hash"}

@@ -353,10 +353,14 @@ Plan plan_gemm(int64_t batch, int64_t m, int64_t n, int64_t k, bool a_kcontig, b
     if (s > max_s) s = max_s;
     if (s > 64) s = 64;
     if (s > 1) {
-      int64_t chunk = (k + s - 1) / s;
-      chunk = (chunk + 63) / 64 * 64;
-      best.splits = (int)((k + chunk - 1) / chunk);
-      best.kchunk = chunk;
+      const int64_t chunk = chunk_of(k, s), sp = (k + chunk - 1) / chunk;
+      // C192 from three quarters of the CUs on: not where its partial sums cost
+      // more than the second block per CU gains (2000 x 2243 at K = 2304 36.2 us,
+      // 43.6 in two splits; but 4393 x 2216 at K = 2275 75.0 and 69.9)
+      if (best.cfg != 2 || tiles < kCUs * 3 / 4 ||
+          plan_time(rounds_of(2, tiles * sp), chunk, sp, batch * m * n) <
+              1.05 * plan_time(rounds_of(2, tiles), k, 1, 0))
+        best.splits = (int)sp, best.kchunk = chunk;
     }
   }
   // Over a very long K a round of C256W takes 1.4 units against the others'
