@@ -142,6 +142,13 @@ def test_splits_of_three_quarters_of_a_round(both, m, n, k, tile, splits):
     assert (tile, splits) in _plan(both[1], "NT", m, n, k)
 
 
+@pytest.mark.parametrize("m,n,k,tile,splits", [(816, 1384, 8192, 128, 6), (4424, 320, 14520, 128, 4), (1500, 1400, 20008, 256, 6)])
+def test_long_k_plans(both, m, n, k, tile, splits):
+    """Splits over a long K go to the 256x256 tiles of four waves where each is long
+    enough and they save enough."""
+    assert (tile, splits) in _plan(both[1], "NT", m, n, k)
+
+
 def test_every_entry_point_is_native(both):
     slow = {name for name in ek.SIGNATURES if getattr(both[1], name).__class__ is not len.__class__}
     assert slow == {"mi355x_abi_version", "mi355x_last_error", "mi355x_target", "mi355x_source_hash"}

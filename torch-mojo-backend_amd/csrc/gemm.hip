@@ -366,17 +366,19 @@ Plan plan_gemm(int64_t batch, int64_t m, int64_t n, int64_t k, bool a_kcontig, b
   // Over a very long K a round of C256W takes 1.4 units against the others'
   // model (50257 into 768 columns, us, before / C256W: 16384 rows C192 1386 /
   // 1268, in four splits 1211; 8192 rows C192 977 / in two splits 660; 2048 rows
-  // C128 in 5 splits 204 / in ten 180; but 1000 rows C128 in 10 splits 95 / in
-  // sixteen 112).
+  // C128 in 5 splits 204 / in ten 180).  It has to save a fifth by the model, and
+  // a split to be 3072 long: four waves start and end a tile slowly (811 x 1382
+  // at K = 8192 in ten splits 44.9 us, C128 in six 36.9; 4421 x 315 at K = 14518 in
+  // seven 79.1, C128 in four 65.9).
   if (a_kcontig && k >= 8192 && m >= 256 && n >= 256 && best.cfg != 4 && !forced) {
     const double r = best.cfg == 3 ? 1.4 * (double)((tiles * best.splits + kCUs - 1) / kCUs)
                                    : rounds_of(best.cfg, tiles * best.splits);
-    double tbest = plan_time(r, best.kchunk, best.splits, batch * m * n);
+    double tbest = 0.8 * plan_time(r, best.kchunk, best.splits, batch * m * n);
     const double whole = plan_time(1.4 * (double)((t256 + kCUs - 1) / kCUs), k, 1, 0);
     for (int64_t sp = 1; sp <= 10; ++sp) {
       const int64_t chunk = chunk_of(k, sp);
       const double t = plan_time(1.4 * (double)((t256 * sp + kCUs - 1) / kCUs), chunk, sp, batch * m * n);
-      if (t < tbest && (sp == 1 || t < 0.85 * whole)) tbest = t, best = Plan{3, (int)((k + chunk - 1) / chunk), chunk};
+      if (t < tbest && (sp == 1 || (t < 0.85 * whole && chunk >= 3072))) tbest = t, best = Plan{3, (int)((k + chunk - 1) / chunk), chunk};
     }
   }
   return best;
