@@ -301,15 +301,18 @@ Plan plan_gemm(int64_t batch, int64_t m, int64_t n, int64_t k, bool a_kcontig, b
   // of a single round empty (1536 x 3072 at K = 16384: 288 C128 tiles 233 us, 72
   // in three splits 160).  Splits have to save 15% by the model, which leaves
   // out the burst of the partial sums (8192 x 3072 at K = 8192: 400 us in one,
-  // 433 in two).  Smaller outputs take split-K C128, with half the splits
+  // 433 in two).  A k-contiguous (or packed) B may take C192 below a
+  // round of C256 (8027 x 1536 at K = 8192 205 us, in C128 243; 6790 x 1713 at K =
+  // 4608 114 and 126).  Smaller outputs take split-K C128, with half the splits
   // (768 x 768 at K = 16384 33 / 40; 768 x 3072 is 96 / 89 by itself, but a
   // training step of such layers was 0.3 ms slower for the partial sums).
   bool planned = false;
   if (!a_kcontig && m >= 256 && n >= 256 && t128 >= kCUs) {
     const double r0 = t256 >= kCUs ? 1e30 : rounds_of(0, t128), r1 = rounds_of(1, t256);
-    const double whole = plan_time(r0 < r1 ? r0 : r1, k, 1, 0);
+    const double r2 = b_kcontig && t256 < kCUs && t192 >= fill ? rounds_of(2, t192) : 1e30;
+    const double r = r2 < r0 && r2 < r1 ? r2 : r0 < r1 ? r0 : r1, whole = plan_time(r, k, 1, 0);
     double tbest = whole;
-    best = Plan{r0 < r1 ? 0 : k >= 2048 ? 3 : 1, 1, k};
+    best = Plan{r == r2 ? 2 : r == r0 ? 0 : k >= 2048 ? 3 : 1, 1, k};
     for (int64_t sp = 2; sp <= 4 && k / sp >= 512; ++sp) {
       const int64_t chunk = chunk_of(k, sp);
       const double t = plan_time(rounds_of(1, t256 * sp), chunk, sp, batch * m * n);
