@@ -41,6 +41,34 @@ def test_gemm_f32_tiles_and_splits(kernels, layout, m, n, k, batch, shift):
         assert bool((err <= bound).all()), (ws_n, float((err / bound).max()))
 
 
+@pytest.mark.parametrize("layout", ["NT", "NN", "TN", "TT"])
+@pytest.mark.parametrize("m,n,k,batch", [(130, 3000, 8, 1), (1000, 1090, 16, 7), (1000, 1090, 16, 8), (1000, 1090, 17, 1),
+                                         (161, 9000, 9, 6), (160, 9000, 9, 6), (3, 24577, 48, 2), (3, 24577, 49, 2),
+                                         (16, 24577, 80, 2), (49160, 17, 48, 1), (1000, 1090, 64, 1), (3000, 1500, 40, 1)])
+def test_gemm_f32_short_k(kernels, layout, m, n, k, batch):
+    """The FMA kernel and the matrix cores on both sides of each line between them,
+    into rows of C at every alignment (an odd stride, a base shifted by one
+    element) with bias: nothing else is written.  A chain of k products is within
+    (k + 2) * 2^-24 of sum |a||b| + |bias|."""
+    gen = torch.Generator().manual_seed(m + n + k)
+    A, B, bias = (torch.randn(*x, generator=gen) for x in ((batch, m, k), (batch, k, n), (n,)))
+    ta = dev((A.transpose(1, 2) if layout[0] == "T" else A).contiguous())
+    tb = dev((B.transpose(1, 2) if layout[1] == "T" else B).contiguous())
+    a_rs, a_cs = (k, 1) if layout[0] == "N" else (1, m)
+    b_rs, b_cs = (n, 1) if layout[1] == "N" else (1, k)
+    args, tbias, ld = (p(ta), a_rs, a_cs, m * k, p(tb), b_rs, b_cs, k * n, 0), dev(bias), n + 3 + n % 2
+    ws_n = lib().mi355x_gemm_workspace_bytes(*args, batch, m, n, k)
+    store = torch.full((1 + batch * m * ld,), 3.0, device="cuda")
+    call("mi355x_gemm", p(store) + 4, 0, ld, m * ld, *args, p(tbias), 0, 0, batch, m, n, k, p(workspace(ws_n)) if ws_n else None,
+         ws_n, None)
+    got = store[1:].view(batch, m, ld)
+    assert float(store[0]) == 3.0 and bool((got[..., n:] == 3.0).all())
+    for i in range(batch):
+        a, b = dev(A[i]).double(), dev(B[i]).double()
+        bound = (k + 2) * 2.0 ** -24 * (a.abs() @ b.abs() + tbias.double().abs())
+        assert bool(((got[i, :, :n].double() - (a @ b + tbias.double())).abs() <= bound).all())
+
+
 def _attention_bounds(q, k, v, do, causal, scale):
     """(O, LSE, dQ, dK, dV) in 64 bits, and what f32 sums and products may be
     off by: u = 2^-24; a score D + 4 roundings of sum |q||k|, a probability

@@ -1,6 +1,8 @@
 // GEMM with f32 operands on v_mfma_f32_16x16x4_f32 (f32 products and sums, as
 // a chain of FMAs; 256 flops per clock and CU, 157 TFLOP/s nominal).
 //
+// A short K over a large output runs on plain FMAs instead (takes_fma).
+//
 // Bound: the MFMA rate.  One MFMA takes 32 cycles and two operand registers,
 // so LDS and L2 traffic are small next to it at a 64x64 wave tile (8 16-byte
 // LDS reads per 64 MFMAs); what has to be kept off its path is load latency
@@ -259,9 +261,10 @@ __global__ void __launch_bounds__(kNT, 2) gemm_f32_tile(GemmArgs g, int tiles_m,
   else if (g.c_dt == MI355X_F32) P = (float*)g.c + bidx * g.c_bs;
   char* Cb = (char*)g.c + bidx * g.c_bs * 2;  // 16-bit C
   const bool beta = g.beta && !g.part;
-  typedef float vec __attribute__((ext_vector_type(F)));
-  // F adjacent columns per lane leave in one store where they are aligned
-  const bool wide = P && !beta && cols[F - 1] < g.n && (rs % F) == 0 && ((uintptr_t)P % (4 * F)) == 0;
+  // F adjacent columns per lane leave in one store, which the hardware splits
+  // where it is not aligned
+  struct Out { float v[F]; };
+  const bool wide = P && !beta && cols[F - 1] < g.n;
 #pragma unroll
   for (int i = 0; i < F; ++i)
 #pragma unroll
@@ -269,10 +272,10 @@ __global__ void __launch_bounds__(kNT, 2) gemm_f32_tile(GemmArgs g, int tiles_m,
       const int64_t row = row0 + F * (4 * lg + e) + i;
       if (row >= g.m) continue;
       if (wide) {
-        vec v;
+        Out out;
 #pragma unroll
-        for (int j = 0; j < F; ++j) v[j] = acc[i][j][e] + bias[j];
-        *(vec*)(P + row * rs + cols[0]) = v;
+        for (int j = 0; j < F; ++j) out.v[j] = acc[i][j][e] + bias[j];
+        *(Out*)(P + row * rs + cols[0]) = out;
         continue;
       }
 #pragma unroll
@@ -284,6 +287,68 @@ __global__ void __launch_bounds__(kNT, 2) gemm_f32_tile(GemmArgs g, int tiles_m,
         else st_any(Cb, g.c_dt, off, beta ? v + ld_any(Cb, g.c_dt, off) : v);
       }
     }
+}
+
+// 64x64 tile by FMAs, 4x4 outputs per thread, in stages of 16 k.
+__global__ void __launch_bounds__(256) gemm_f32_fma(GemmArgs g) {
+  __shared__ float As[16][64 + 4];
+  __shared__ float Bs[16][64 + 4];
+  const int64_t batch = blockIdx.z;
+  const int64_t m0 = (int64_t)blockIdx.y * 64, n0 = (int64_t)blockIdx.x * 64;
+  const float* A = (const float*)g.a + batch * g.a_bs;
+  const float* B = (const float*)g.b + batch * g.b_bs;
+  const int tx = threadIdx.x & 15, ty = threadIdx.x >> 4;
+  float acc[4][4] = {};
+  for (int64_t k0 = 0; k0 < g.k; k0 += 16) {
+    for (int e = threadIdx.x; e < 16 * 64; e += 256) {
+      const int kk = e / 64, r = e % 64;
+      const int64_t gm = m0 + r, gk = k0 + kk, gn = n0 + r;
+      As[kk][r] = (gm < g.m && gk < g.k) ? A[gm * g.a_rs + gk * g.a_cs] : 0.f;
+      Bs[kk][r] = (gn < g.n && gk < g.k) ? B[gk * g.b_rs + gn * g.b_cs] : 0.f;
+    }
+    __syncthreads();
+#pragma unroll
+    for (int kk = 0; kk < 16; ++kk) {
+      float a[4], b[4];
+#pragma unroll
+      for (int i = 0; i < 4; ++i) a[i] = As[kk][ty * 4 + i], b[i] = Bs[kk][tx * 4 + i];
+#pragma unroll
+      for (int i = 0; i < 4; ++i)
+#pragma unroll
+        for (int j = 0; j < 4; ++j) acc[i][j] += a[i] * b[j];
+    }
+    __syncthreads();
+  }
+  void* Cb = (char*)g.c + batch * g.c_bs * (g.c_dt == MI355X_F32 ? 4 : 2);
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    const int64_t row = m0 + ty * 4 + i;
+    if (row >= g.m) continue;
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      const int64_t col = n0 + tx * 4 + j;
+      if (col >= g.n) continue;
+      float v = acc[i][j] + (g.bias ? ld_any(g.bias, g.bias_dt, col) : 0.f);
+      const int64_t off = row * g.c_rs + col;
+      if (g.beta) v += ld_any(Cb, g.c_dt, off);
+      st_any(Cb, g.c_dt, off, v);
+    }
+  }
+}
+
+// Where the FMA kernel is the faster one: up to half of its first stage, and all
+// of it while there are few tiles or thin ones (matrix cores over FMA, geometric
+// means of drawn shapes: up to 256 tiles 1.05 at K <= 2, 1.0 at 9 .. 16; up to 2048
+// 1.33 and 1.14 .. 1.22; 14008 x 1151 at K = 1 26.8 us, on matrix cores 34.9; past
+// 2048 tiles at K = 9 .. 16 0.82 .. 0.98); and many tiles of few rows or columns
+// where its stages of 16 k cover K more closely than those of 32 (28 batches of 1 x
+// 50257 at K = 40 121 us, on matrix cores 187, 4 x 14257 x 2 at K = 41 10.3 and 13.0;
+// up to 32 rows at K = 33 .. 48 FMA takes 0.77 .. 0.91 of the time, at 49 .. 64 1.0
+// .. 1.2).
+bool takes_fma(int64_t batch, int64_t m, int64_t n, int64_t k) {
+  const int64_t tiles = ((m + 63) / 64) * ((n + 63) / 64) * batch, least = m < n ? m : n;
+  if (least <= 32 && tiles >= 3 * kCUs) return k <= 48 || (least <= 16 && k > 64 && k <= 80);
+  return k <= 8 || (k <= 16 && (tiles <= 2048 || least <= 160));
 }
 
 struct PlanF32 {
@@ -303,6 +368,10 @@ PlanF32 plan_f32(int64_t batch, int64_t m, int64_t n, int64_t k) {
   double tbest = 1e30;
   for (int tile = 128; tile >= 64; tile -= 64) {
     const int64_t tiles = ((m + tile - 1) / tile) * ((n + tile - 1) / tile) * batch;
+    // one round of 128 tiles over a short K: a block's start and end take its time
+    // (3906 x 1019 at K = 63 21.3 us, in 64 tiles 15.3)
+    if (tile == 128 && k <= 64 && tiles <= kCUs) continue;
+    if (tile == 64 && tiles >= 1 << 24) continue;  // a launch takes fewer than 2^32 threads
     const double per_k = 2.0 * tile * tile / (tile == 128 ? 440e3 : 375e3);  // us
     for (int64_t sp = 1; sp <= 32 && (sp == 1 || (k / sp >= 128 && tiles < 4 * kCUs)); ++sp) {
       int64_t chunk = (k + sp - 1) / sp;
@@ -360,11 +429,16 @@ bool vec_ok(const void* p, int64_t ld, int64_t bs, int64_t extent) {
 }  // namespace
 
 int64_t gemm_f32_workspace(int64_t batch, int64_t m, int64_t n, int64_t k) {
+  if (takes_fma(batch, m, n, k)) return 0;
   const PlanF32 p = plan_f32(batch, m, n, k);
   return p.splits > 1 ? (int64_t)p.splits * batch * m * n * 4 : 0;
 }
 
 int gemm_f32_launch(GemmArgs g, int64_t batch, void* workspace, int64_t ws_bytes, hipStream_t s) {
+  if (takes_fma(batch, g.m, g.n, g.k)) {
+    gemm_f32_fma<<<dim3(ceil_div(g.n, 64), ceil_div(g.m, 64), (unsigned)batch), kNT, 0, s>>>(g);
+    return check_launch("mi355x_gemm");
+  }
   PlanF32 p = plan_f32(batch, g.m, g.n, g.k);
   if (p.splits > 1 && (!workspace || ws_bytes < (int64_t)p.splits * batch * g.m * g.n * 4))
     p.splits = 1, p.kchunk = g.k;
