@@ -630,7 +630,9 @@ int copy_two_unit(void* dst, int dst_dt, const void* src, int src_dt, const Geo&
   int c = -1;
   for (int i = 0; i < d; ++i)
     if (g.st[1][i] == 1) c = i;
-  if (c < 0 || g.st[0][d] != 1 || g.st[1][d] == 1 || g.shape[d] < 8 || g.shape[c] < 16) return -1;
+  if (c < 0 || g.st[0][d] != 1 || g.st[1][d] == 1 || g.shape[d] < 8 || g.shape[c] < 16 ||
+      g.shape[d] * g.shape[c] < 256)
+    return -1;
   TwoUnit t{};
   t.nd = g.shape[d], t.ns = g.shape[c], t.dst_s = g.st[0][c], t.src_d = g.st[1][d];
   t.tiles_s = (t.ns + 63) / 64, t.tiles_d = (t.nd + 63) / 64, t.tiles = t.tiles_s * t.tiles_d;
