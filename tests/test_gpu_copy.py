@@ -53,3 +53,16 @@ def test_cast_every_order(kernels, src_dtype, dst_dtype, shape):
         dst = torch.zeros([shape[i] for i in pd], dtype=dst_dtype, device="cuda").permute([pd.index(i) for i in range(3)])
         _copy(dst, src)
         assert torch.equal(dst, src.to(dst_dtype)), (ps, pd)
+
+
+@pytest.mark.parametrize("rows,row_bytes", [(1, 16384), (3, 16384 * 3), (5, 16384 * 2 + 16), (16, 16368), (2047, 32784),
+                                            (2048, 32784)])
+def test_copy_few_long_rows(kernels, rows, row_bytes):
+    """Rows cut into pieces of 16 KB (below 2048 of them) and rows that a wave takes
+    whole, from a strided source and from one row broadcast; nothing else is written."""
+    n, wide = row_bytes // 4, row_bytes // 4 + 8
+    src = torch.randn(rows, wide, device="cuda")
+    for view in (src[:, 4:4 + n], src[:1, :n].expand(rows, n)):
+        store = torch.full((rows, wide), 7.0, device="cuda")
+        _copy(store[:, :n], view)
+        assert torch.equal(store[:, :n], view) and bool((store[:, n:] == 7.0).all())

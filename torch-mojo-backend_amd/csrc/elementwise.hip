@@ -477,15 +477,17 @@ __global__ void __launch_bounds__(kThreads) cast_bf16_f32(float* __restrict__ ou
   }
 }
 // Same-dtype copy of `rows` rows of `row_bytes` (16-byte multiples) between
-// row strides (slices, concatenation): one 64-lane wave per row.
+// row strides (slices, concatenation): one 64-lane wave per row, or, of few rows,
+// per `seg` bytes of one (16 rows of 4.9 MB: a wave a row 1229 us).
 __global__ void __launch_bounds__(kThreads) copy_rows_b128(uint8_t* __restrict__ dst, int64_t dst_rs,
                                                            const uint8_t* __restrict__ src, int64_t src_rs,
-                                                           int64_t rows, int64_t row_bytes) {
+                                                           int64_t rows, int64_t row_bytes, int64_t seg, int segs) {
   const int lane = threadIdx.x & 63;
-  const int64_t nv = row_bytes / 16;
-  for (int64_t r = (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6); r < rows; r += (int64_t)gridDim.x * 4) {
-    const uint4* s = (const uint4*)(src + r * src_rs);
-    uint4* d = (uint4*)(dst + r * dst_rs);
+  for (int64_t t = (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6); t < rows * segs; t += (int64_t)gridDim.x * 4) {
+    const int64_t r = segs == 1 ? t : t / segs, at = (t - r * segs) * seg;
+    const int64_t nv = min(seg, row_bytes - at) / 16;
+    const uint4* s = (const uint4*)(src + r * src_rs + at);
+    uint4* d = (uint4*)(dst + r * dst_rs + at);
     for (int64_t k = lane; k < nv; k += 64) d[k] = s[k];
   }
 }
@@ -737,10 +739,13 @@ extern "C" int mi355x_copy(void* dst, int dst_dtype, const int64_t* dst_strides,
     const int64_t chunks = n * es / 16;
     const bool few = chunks < (int64_t)1 << 31;  // 32-bit index and grid stride
     if (wide && g.ndim == 2 && (rb >= 1024 || !few)) {
-      int64_t blocks = (g.shape[0] + 3) / 4;
+      // fewer waves than two blocks per CU: 16 KB of a row each
+      const int64_t seg = g.shape[0] < 2048 ? 16384 : rb;
+      const int segs = (int)((rb + seg - 1) / seg);
+      int64_t blocks = (g.shape[0] * segs + 3) / 4;
       if (blocks > 65536) blocks = 65536;
       copy_rows_b128<<<(unsigned)blocks, kThreads, 0, s>>>((uint8_t*)dst, g.st[0][0] * es, (const uint8_t*)src,
-                                                            g.st[1][0] * es, g.shape[0], rb);
+                                                            g.st[1][0] * es, g.shape[0], rb, seg, segs);
       return check_launch("mi355x_copy");
     }
     if (wide && few) {
