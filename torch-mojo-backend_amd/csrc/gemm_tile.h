@@ -46,12 +46,10 @@ extern __shared__ __attribute__((aligned(16))) char gemm_smem[];
 namespace mi {
 namespace {
 
-// Row swizzle of a k-contiguous tile with BK-element (2*BK-byte) rows: row r
-// stores its 16-byte chunk c in slot c ^ rswz(r).  A fragment read (16 rows
-// at one chunk) then covers every bank once: BK = 64, 8 chunks, rows paired
-// by (r >> 1); BK = 32, 4 chunks, rows grouped by (r >> 2).
-template <int BK>
-__device__ __forceinline__ int rswz(int r) { return BK == 64 ? ((r >> 1) & 7) : ((r >> 2) & 3); }
+// Row swizzle of a k-contiguous tile with 128-byte rows (64 k): row r stores its
+// 16-byte chunk c in slot c ^ rswz(r).  A fragment read (16 rows at one chunk)
+// then covers every bank once: 8 chunks, rows paired by (r >> 1).
+__device__ __forceinline__ int rswz(int r) { return (r >> 1) & 7; }
 
 // k-contiguous operand tile: ROWS rows x BK k, loaded by NT threads, one
 // 1 KB instruction per RPI rows.  Thread (wave w, lane l) handles rows
@@ -60,6 +58,7 @@ __device__ __forceinline__ int rswz(int r) { return BK == 64 ? ((r >> 1) & 7) : 
 // operand's end reload its last row (their results are never stored).
 template <int ROWS, int NT, int BK>
 struct TileLoad {
+  static_assert(BK == 64, "rswz");
   static constexpr int CPR = BK / 8;    // 16-byte chunks per row
   static constexpr int RPI = 64 / CPR;  // rows per 1 KB instruction
   static constexpr int WAVES = NT / 64;
@@ -71,7 +70,7 @@ struct TileLoad {
   __device__ __forceinline__ void init(const char* base, int64_t ld_bytes, int64_t row0, int64_t rows) {
     const int lane = threadIdx.x & 63, wave = wave_id();
     const int r = wave * RPI + lane / CPR;
-    chunk = (lane % CPR) ^ rswz<BK>(r);
+    chunk = (lane % CPR) ^ rswz(r);
 #pragma unroll
     for (int it = 0; it < ITERS; ++it) {
       int64_t row = row0 + r + it * RPI * WAVES;
@@ -395,7 +394,7 @@ __device__ __forceinline__ typename Mfma<T>::frag read_frag(const char* tile, in
   typedef typename Mfma<T>::frag frag;
   const int lane = threadIdx.x & 63, lr = lane & 15, lg = lane >> 4;
   if constexpr (K_CONTIG) {
-    return *(const frag*)(tile + (r0 + lr) * 128 + ((ks * 4 + lg) ^ rswz<64>(lr)) * 16);
+    return *(const frag*)(tile + (r0 + lr) * 128 + ((ks * 4 + lg) ^ rswz(lr)) * 16);
   } else {
     frag f[1];
     mn_frags<T, ROWS, 1>(tile, r0, ks, f);
@@ -404,8 +403,10 @@ __device__ __forceinline__ typename Mfma<T>::frag read_frag(const char* tile, in
 }
 
 // c += a b on accumulators that stay where they are: given the builtin, the
-// compiler moves 256 of them about between the MFMAs of a loop.  The hazard
-// that this hides from it, reading c too soon after, is settle_acc's.
+// compiler moves 256 of them about between the MFMAs of a loop.  It does not see
+// that c is an MFMA's result, which other instructions may read only 10 states
+// later: nothing may read or copy an accumulator before the s_nops that end
+// wide_loop.
 typedef int i32x4 __attribute__((ext_vector_type(4)));
 __device__ __forceinline__ void mma_acc(f32x4& c, const Mfma<bf16>::frag& a, const Mfma<bf16>::frag& b) {
   asm volatile("v_mfma_f32_16x16x32_bf16 %0, %1, %2, %0"
@@ -426,8 +427,9 @@ __device__ __forceinline__ void mma_acc(f32x4& c, const Mfma<f16>::frag& a, cons
 // transposed operands.
 // Against C256 (us): 8192^3 917 -> 869, dX 1074 -> 927, dW 1110 -> 994; 50257
 // columns dX 16384 rows 1468 -> 1268 (C192 1386), dW 1275 -> 1160; 16384 x
-// 4096 at K = 4096 471 -> 461; but at K = 768 83 -> 86 and 74 -> 79: four waves
-// fill and drain a tile more slowly than eight.
+// 4096 at K = 4096 471 -> 461; but at K = 768 83 -> 86 and 74 -> 79 (the only wave
+// of a SIMD zeroes 256 accumulators and ends with 64 s_nops; what share of that
+// they have is not measured).
 template <typename T, typename C, bool KT, bool A_K, bool B_K, typename LA, typename LB, int TM, int TN>
 __device__ __forceinline__ void wide_loop(const LA& la, const LB& lb, f32x4 (&acc)[TM][TN], char* lds, int64_t kbeg,
                                           int64_t kend, int wm, int wn) {
@@ -594,7 +596,7 @@ __global__ void __launch_bounds__(64 * TileCfg<CFG>::WGM * TileCfg<CFG>::WGN, Ti
     }
   }
   // k-contiguous fragment rows (.. + lr) share the swizzle of lr
-  const int sw = rswz<BK>(lr);
+  const int sw = rswz(lr);
   const int rs_slots = g.part ? g.tiles_n * C::WGN : 1;
   const int rs_slot = g.part ? (int)tn * C::WGN + wn : 0;
   const bool rs_on = RS && (g.part || (tn == 0 && wn == 0));
