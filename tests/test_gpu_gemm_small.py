@@ -1,5 +1,5 @@
-"""The 64x64 GEMM tiles (outputs too small to fill the CUs with larger ones),
-through the C ABI, against 64-bit results."""
+"""The 16-bit GEMM's tiles, plans and stores through the C ABI, against 64-bit
+results."""
 
 import pytest
 import torch
@@ -41,11 +41,23 @@ def test_gemm_64_tiles(kernels, dtype, layout, m, n, k, batch):
 @pytest.mark.parametrize("c_dtype,flags", [(torch.bfloat16, 0), (torch.float16, 0), (torch.float32, 0), (torch.float32, 2),
                                            (torch.bfloat16, 1)])
 def test_gemm_stores_at_any_alignment(kernels, m, n, layout, c_dtype, flags):
-    """Partial tiles of each block configuration into rows of C at every
-    alignment (odd row stride, a base shifted by one element): every element
-    of C right, nothing else written.  k = 64 sums of exact products, rounded
-    once to the output type (and through bf16 with ROUND)."""
-    k, ld, shift = 64, n + 3 + n % 2, 1
+    """Partial tiles (64x64, 128x128 and twice 128x192) into rows of C at every
+    alignment."""
+    _stores_at_any_alignment(m, n, 64, layout, c_dtype, flags)
+
+
+@pytest.mark.parametrize("k", [64, 2056])
+@pytest.mark.parametrize("c_dtype,flags", [(torch.bfloat16, 0), (torch.float32, 0), (torch.float32, 2), (torch.bfloat16, 1)])
+def test_gemm_wide_tiles_store_at_any_alignment(kernels, k, c_dtype, flags):
+    """The same from 256x256 tiles: of eight waves, and (K = 2056) of four."""
+    _stores_at_any_alignment(4090, 4093, k, "NT", c_dtype, flags)
+
+
+def _stores_at_any_alignment(m, n, k, layout, c_dtype, flags):
+    """C into an odd row stride and a base shifted by one element: every element
+    of C right, nothing else written.  Sums of k exact products, rounded once to
+    the output type (and through bf16 with ROUND)."""
+    ld, shift = n + 3 + n % 2, 1
     gen = torch.Generator().manual_seed(m + n)
     A, B, bias = (torch.randn(*s, generator=gen).bfloat16() for s in ((m, k), (k, n), (n,)))
     ta, tb, tbias = dev(A), dev((B.t() if layout[1] == "T" else B).contiguous()), dev(bias)
@@ -97,9 +109,9 @@ def test_gemm_groups_of_tile_rows(kernels, dtype, layout, m, n, k, batch):
 @pytest.mark.parametrize("m,n,k,rows", [(520, 300, 8200, False), (2100, 776, 8192, False), (3600, 3850, 2048, False),
                                         (1540, 3090, 4104, True), (1540, 3090, 4160, False)])
 def test_gemm_long_k(kernels, dtype, layout, m, n, k, rows):
-    """256x256 tiles of four waves: whole K and splits, one to three stages
-    past the ring's length, a ragged last stage, edges of the tile, and the
-    row sums that take eight waves instead."""
+    """Long K in each plan around the 256x256 tiles of four waves (which take the
+    whole K of 3600 x 3850): 64x64 tiles and 128x128 tiles in splits, 128x192 tiles
+    whole and in two splits, ragged last stages, and row sums."""
     gen = torch.Generator().manual_seed(m + 3 * n + k)
     n8, m8 = (n + 7) // 8 * 8, (m + 7) // 8 * 8  # rows in place: strides of whole 16 bytes
     A, B = (torch.randn(*s, generator=gen).to(dtype) for s in ((m8, k), (k, n8)))
@@ -141,6 +153,37 @@ def test_gemm_long_k_ends(kernels, layout, k):
     assert bool(((c.double() - a @ b).abs() <= (k + 3) * 2.0 ** -23 * (a.abs() @ b.abs())).all())
 
 
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("layout,m,n,k,splits,batch", [("NT", 1500, 1400, 20008, 6, 1), ("NN", 1500, 1400, 20000, 6, 1),
+                                                       ("NN", 1000, 1100, 20008, 6, 2), ("TN", 1500, 2900, 8200, 3, 1),
+                                                       ("TT", 1500, 2900, 8200, 3, 1), ("TN", 1500, 2900, 6144, 3, 1),
+                                                       ("TT", 1500, 2900, 6152, 3, 1)])
+@pytest.mark.parametrize("rows", [False, True])
+def test_gemm_wide_tiles_in_splits(kernels, dtype, layout, m, n, k, splits, batch, rows):
+    """K splits of the 256x256 tiles (an odd count of 128-wide columns tells their
+    row-sum slots from the smaller tiles', so that the workspace's size names the
+    plan), the last split shorter and ragged or whole: of four waves, and with row
+    sums of eight."""
+    n8, m8, up = (n + 7) // 8 * 8, (m + 7) // 8 * 8, lambda v: (v + 255) // 256 * 256
+    gen = torch.Generator().manual_seed(m + 3 * n + k)
+    A, B = (torch.randn(batch, *s, generator=gen).to(dtype) for s in ((m8, k), (k, n8)))
+    ta = dev((A.transpose(1, 2) if layout[0] == "T" else A).contiguous())
+    tb = dev((B.transpose(1, 2) if layout[1] == "T" else B).contiguous())
+    a_rs, a_cs = (k, 1) if layout[0] == "N" else (1, m8)
+    b_rs, b_cs = (n8, 1) if layout[1] == "N" else (1, k)
+    args = (p(ta), a_rs, a_cs, m8 * k, p(tb), b_rs, b_cs, k * n8)
+    ws_n = lib().mi355x_gemm_workspace_bytes(*args, CODE[dtype], batch, m, n, k)
+    assert ws_n == up(splits * batch * m * n * 4) + up(splits * batch * -(-n // 256) * 4 * m * 4)
+    ws, c = workspace(ws_n), torch.full((batch, m, n), float("nan"), device="cuda")
+    sums = torch.full((batch, m), float("nan"), device="cuda") if rows else None
+    call("mi355x_gemm_ex", p(c), 0, n, m * n, *args, CODE[dtype], None, 0, 0, p(sums), 0, batch, m, n, k, p(ws), ws_n, None)
+    for i in range(batch):
+        a, b, u = dev(A[i, :m]).double(), dev(B[i, :, :n]).double(), (k + 3) * 2.0 ** -23
+        assert bool(((c[i].double() - a @ b).abs() <= u * (a.abs() @ b.abs())).all())
+        if rows:
+            assert bool(((sums[i].double() - a.sum(1)).abs() <= u * a.abs().sum(1)).all())
+
+
 @pytest.mark.parametrize("layout", ["TN", "TT"])
 @pytest.mark.parametrize("k", [72, 520, 1984])
 def test_gemm_row_sums_of_whole_wide_tiles(kernels, layout, k):
@@ -153,8 +196,9 @@ def test_gemm_row_sums_of_whole_wide_tiles(kernels, layout, k):
     b_rs, b_cs = (n, 1) if layout[1] == "N" else (1, k)
     args = (p(ta), 1, 4096, 0, p(tb), b_rs, b_cs, 0)
     ws_n = lib().mi355x_gemm_workspace_bytes(*args, 1, 1, m, n, k)
+    ws = workspace(ws_n)
     c, sums = torch.full((m, n), float("nan"), device="cuda"), torch.full((m,), float("nan"), device="cuda")
-    call("mi355x_gemm_ex", p(c), 0, n, 0, *args, 1, None, 0, 0, p(sums), 0, 1, m, n, k, p(workspace(ws_n)), ws_n, None)
+    call("mi355x_gemm_ex", p(c), 0, n, 0, *args, 1, None, 0, 0, p(sums), 0, 1, m, n, k, p(ws), ws_n, None)
     a, b, u = dev(A[:m]).double(), dev(B).double(), (k + 3) * 2.0 ** -23
     assert bool(((c.double() - a @ b).abs() <= u * (a.abs() @ b.abs())).all())
     assert bool(((sums.double() - a.sum(1)).abs() <= u * a.abs().sum(1)).all())
