@@ -38,6 +38,10 @@ def test_errors_stay_errors(mojo):
     for call in (lambda: m.view(5, 5), lambda: m.view(-1, -1), lambda: m.view(-1, 0), lambda: m.t().view(24)):
         with pytest.raises(RuntimeError):
             call()
+    for call, text in ((lambda: torch.as_strided(m, (2, 2), (1,)), "dimensionality of sizes"),
+                       (lambda: m.split([-1, 5]), "non-negative")):
+        with pytest.raises(RuntimeError, match=text):
+            call()
     with pytest.raises(NotImplementedError):
         TorchMojoTensor._alloc((1,) * 9, torch.float32, 0)
     with pytest.raises(RuntimeError):

@@ -324,6 +324,14 @@ int ints_of(PyObject* o, int64_t* v) {
   return (int)n;
 }
 
+// The same for strides of a shape with nd dimensions, as torch reports it.
+bool strides_of(PyObject* o, int64_t* v, int nd) {
+  const int n = ints_of(o, v);
+  if (n >= 0 && n != nd)
+    PyErr_Format(PyExc_RuntimeError, "dimensionality of sizes (%d) must match dimensionality of strides (%d)", nd, n);
+  return n == nd;
+}
+
 PyObject* tuple_of(const int64_t* v, int n) {
   PyObject* t = PyTuple_New(n);
   if (!t) return nullptr;
@@ -390,10 +398,7 @@ PyObject* make(PyObject*, PyObject* const* a, Py_ssize_t n) {
   }
   int64_t shape[kMaxRank], strides[kMaxRank];
   const int nd = ints_of(a[2], shape);
-  if (nd < 0 || ints_of(a[3], strides) != nd) {
-    if (!PyErr_Occurred()) PyErr_SetString(PyExc_ValueError, "shape and strides differ in length");
-    return nullptr;
-  }
+  if (nd < 0 || !strides_of(a[3], strides, nd)) return nullptr;
   int64_t numel;
   if (!product(shape, nd, &numel)) return nullptr;
   const bool c = a[7] == Py_None ? contiguous(shape, strides, nd) : PyObject_IsTrue(a[7]) == 1;
@@ -541,10 +546,7 @@ PyObject* view_of(PyObject*, PyObject* const* a, Py_ssize_t n) {
   if (!read(a[0], &m)) return not_mojo();
   int64_t shape[kMaxRank], strides[kMaxRank], off;
   const int nd = ints_of(a[1], shape);
-  if (nd < 0 || ints_of(a[2], strides) != nd || !as_i64(a[3], &off)) {
-    if (!PyErr_Occurred()) PyErr_SetString(PyExc_ValueError, "shape and strides differ in length");
-    return nullptr;
-  }
+  if (nd < 0 || !strides_of(a[2], strides, nd) || !as_i64(a[3], &off)) return nullptr;
   int64_t delta;
   if (__builtin_sub_overflow(off, (int64_t)PyLong_AsLongLong(m.offset), &delta)) {
     overflow("the offset of a view");

@@ -646,6 +646,9 @@ def fast_aten_split_with_sizes(self, split_sizes, dim=0):
         raise RuntimeError("split_with_sizes expects split_sizes to sum exactly to the dim size")
     outs, start, narrow = [], 0, _host().narrow
     for s in split_sizes:
+        if s < 0:
+            raise RuntimeError("split_with_sizes expects split_sizes have only non-negative entries, but got"
+                               f" split_sizes={list(split_sizes)}")
         outs.append(narrow(t, d, start, s))
         start += s
     return outs
