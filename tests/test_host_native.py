@@ -81,6 +81,19 @@ def test_views_past_64_bits_are_refused(mojo):
     assert empty.view(2 ** 40, 0).shape == (2 ** 40, 0) and m.expand(2 ** 40, 4, 6).shape[0] == 2 ** 40
 
 
+def test_operands_of_other_sizes_are_refused(mojo):
+    """A bias that does not broadcast to the product raises, as on the CPU: its
+    elements past the end are not read."""
+    x, w = torch.ones(3, 6).to("mojo"), torch.ones(6, 6).to("mojo")
+    for shape in ((4,), (4, 1), (3, 5), (2, 3, 6)):
+        b = torch.ones(shape)
+        cpu, dev = (lambda: torch.addmm(b, x.cpu(), w.cpu())), (lambda: torch.addmm(b.to("mojo"), x, w))
+        for call in (cpu, dev, lambda: torch.nn.functional.linear(x, w, b.to("mojo")),
+                     lambda: torch.addmm(b.to("mojo"), x, w, beta=2.0)):
+            with pytest.raises(RuntimeError):
+                call()
+
+
 @pytest.fixture(scope="module")
 def both():
     return ek._load(), ek._NativeLibrary(ek._load())

@@ -143,12 +143,15 @@ def _broadcast_strides(t: MT, shape) -> tuple[int, ...]:
     out = []
     for i in range(nd):
         j = i - pad
-        if j < 0 or t._shape[j] == 1 and shape[i] != 1:
+        if j < 0 or t._shape[j] == 1:
             out.append(0)
-        elif t._shape[j] == 1:
-            out.append(0)
+        elif t._shape[j] != shape[i]:
+            raise RuntimeError(f"The size of tensor a ({shape[i]}) must match the size of tensor b ({t._shape[j]}) at"
+                               f" non-singleton dimension {i}")
         else:
             out.append(t._strides[j])
+    if pad < 0 and any(n != 1 for n in t._shape[:-pad]):
+        raise RuntimeError(f"shape {tuple(t._shape)} cannot be broadcast to {tuple(shape)}")
     return tuple(out)
 
 
