@@ -94,6 +94,25 @@ def test_operands_of_other_sizes_are_refused(mojo):
                 call()
 
 
+def test_views_stay_in_their_storage(mojo):
+    """as_strided past the storage, with a negative stride or offset, and permute
+    with a dimension twice or left out raise, as on the CPU."""
+    m = torch.arange(24.0).reshape(4, 6).to("mojo")
+    for args in (((4, 6), (6, 1), 1), ((2, 2), (1, 23), 0), ((2,), (-1,), 3), ((2,), (1,), -1), ((25,), (1,)), ((1,), (1,), 24),
+                 ((-1,), (1,))):
+        for t in (m, m.cpu()):
+            with pytest.raises(RuntimeError):
+                torch.as_strided(t, *args)
+    for dims in ((0, 0), (0,), (1, 0, 1)):
+        for t in (m, m.cpu()):
+            with pytest.raises(RuntimeError):
+                t.permute(dims)
+    for t, args in ((m, ((3, 4), (2, 3), 5)), (m[2:], ((2, 2), (1, 2))), (m[2:], ((4, 6), (6, 1), 0)), (m, ((0, 9), (1, 1), 99)),
+                    (m.t(), ((24,), (1,)))):
+        assert torch.equal(torch.as_strided(t, *args).cpu(), torch.as_strided(m.cpu(), *args[:2], args[2] if len(args) > 2
+                                                                              else t.storage_offset()))
+
+
 @pytest.fixture(scope="module")
 def both():
     return ek._load(), ek._NativeLibrary(ek._load())

@@ -546,7 +546,16 @@ def fast_aten__reshape_alias(self, size, stride):
 def fast_aten_as_strided(self, size, stride, storage_offset=None):
     t = _require(self)
     off = t._offset if storage_offset is None else int(storage_offset)
-    return MT._view_of(t, tuple(size), tuple(stride), off)
+    size, stride = tuple(size), tuple(stride)
+    if any(s < 0 for s in stride) or any(n < 0 for n in size) or off < 0:
+        raise RuntimeError(f"as_strided: negative size, stride or offset ({size}, {stride}, {off})")
+    if 0 not in size:
+        start = t._ptr - t._offset * t._itemsize - t._holder.data_ptr()  # of the storage, in the holder
+        end = off + 1 + sum((n - 1) * s for n, s in zip(size, stride))
+        if start + end * t._itemsize > t._holder.numel():
+            raise RuntimeError(f"setStorage: sizes {size}, strides {stride} and storage offset {off} are out of bounds for"
+                               f" storage of size {t._holder.numel() - start}")
+    return MT._view_of(t, size, stride, off)
 
 
 def fast_aten_alias(self):
@@ -571,6 +580,8 @@ def fast_aten_permute(self, dims):
     t = _require(self)
     nd = len(t._shape)
     dims = [_norm_dim(d, nd) for d in dims]
+    if len(dims) != nd or len(set(dims)) != nd:
+        raise RuntimeError(f"permute: {dims} is no order of {nd} dimensions")
     return MT._view_of(t, [t._shape[d] for d in dims], [t._strides[d] for d in dims], t._offset)
 
 
