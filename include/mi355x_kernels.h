@@ -501,7 +501,7 @@ int mi355x_foreach_apply(int op, void* const* a, const void* const* b,
  * B element at b + b*b_bs + k*b_rs + n*b_cs (b_rs == 1 or b_cs == 1),
  * C element at c + b*c_bs + m*c_rs + n (rows contiguous).
  * ab_dtype: F32, BF16 or F16 (A and B share it); c_dtype and bias_dtype:
- * F32/BF16/F16.  Accumulates in f32, on MFMA.  beta == 1 adds the
+ * F32/BF16/F16.  Accumulates in f32, on MFMA (f32 of a short K: on FMAs).  beta == 1 adds the
  * existing C (accumulate), beta == 0 overwrites. */
 /* Workspace for the call with these operands (split-K partials, and packed
  * copies of operands that cannot be read in place; f32 operands: the partials
